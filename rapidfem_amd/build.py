@@ -18,7 +18,7 @@ CSRC = os.path.join(PKG, "csrc")
 OUT_DIR = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "librfhip.so")
 
-HIP_SOURCES = ["rfhip_api.hip", "rfhip_plain.hip", "rfhip_fused.hip", "rfhip_vec.hip", "rfhip_debye.hip",
+HIP_SOURCES = ["rfhip_api.hip", "rfhip_plain.hip", "rfhip_fused.hip", "rfhip_quad.hip", "rfhip_vec.hip", "rfhip_debye.hip",
                "rfhip_sparse.hip", "rfhip_xfer.hip", "rfhip_mlp.hip", "rfhip_noalloc.hip"]
 CXX_SOURCES = ["host_builder.cpp", "krylov_host.cpp"]
 

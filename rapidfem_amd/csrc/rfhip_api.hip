@@ -165,16 +165,21 @@ void build_plain(rfhip_op *op, const rfhip_op_desc &d) {
   dv.port = op->port.as<int>();
   dv.perm = op->perm.as<int>();
 }
-// Stage-kernel variant an operator starts with: the fastest per order and
-// register form in a sweep of every variant over LSERK4 steps on MI355X
-// (pulse boxes of 1.3M / 393k / 324k / 96k tets at N = 1..4; N = 2 and the
-// FP64 registers at N = 3 again on 768k / 324k tets once k_fused11 fitted
-// those cases to 2 waves per SIMD, N = 4 on the 998k-tet cavity once
-// k_fused9's LDS fitted two blocks per CU). autotune re-picks on the
-// operator's own mesh.
-int default_variant(int order, int form) {
+// Stage-kernel variant an operator starts with. With FP64 registers k_quad
+// (variant 9) where its table exists: on MI355X it is the fastest at every
+// order from 48 tets to the largest meshes swept (us per stage, fastest other
+// variant against k_quad: 1,296 tets 5.6 / 3.9, 7.6 / 5.4, 9.4 / 8.4,
+// 15.4 / 15.1 at N = 1..4; 1.3M / 768k / 324k / 384k tets 288 / 271,
+// 484 / 350, 416 / 290, 1232 / 687). With compressed registers, whose
+// rounding of p to f32 turns any other order of the sums into differences
+// of the size of that rounding within a few dozen stages, the variants they
+// have always started with (the fastest of the rest per order: pulse boxes of
+// 1.3M / 393k / 324k / 96k tets at N = 1..4), also for operators without the
+// table. autotune re-picks on the operator's own mesh.
+int default_variant(int order, int form, const StageArgs &a) {
   if (form_vmf(form)) return 1;
   const bool c = form == RFHIP_FORM_FUSED_F64C;
+  if (!c && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
   switch (order) {
     case 1: return c ? 7 : 5;
     case 2: return c ? 7 : 6;
@@ -376,6 +381,20 @@ void build_fused(rfhip_op *op, const rfhip_op_desc &d) {
   std::vector<double> clane;
   const bool has_clane = clane_pack(np, d.face_nodes, D, d.lift, clane);
   if (has_clane) upload(op->clane, clane.data(), clane.size(), s);
+  // k_quad (variant 9) on the same element: its fragments and packed node
+  // rows. It addresses vectors by 32-bit byte offsets.
+  std::vector<double> quad;
+  std::vector<uint8_t> quad_nodes;
+  const bool has_quad = has_clane && 48 * (uint64_t)np * (uint64_t)K < ((uint64_t)1 << 32);
+  if (has_quad) {
+    quad_pack(np, D, d.lift, quad);
+    quad_nodes.assign(100 * 16, 0);
+    for (int r = 0; r < 100; ++r)
+      for (int m = 0; m < nfp; ++m)
+        quad_nodes[16 * r + m] = (uint8_t)(r < 96 ? nbr_node[(size_t)r * nfp + m] : d.face_nodes[(r - 96) * nfp + m]);
+    upload(op->quad, quad.data(), quad.size(), s);
+    upload(op->quad_nodes, quad_nodes.data(), quad_nodes.size(), s);
+  }
   upload(op->jinv64, d.jinv, 9 * (size_t)K, s);
   upload(op->fcode, fcode.data(), fcode.size(), s);
   upload(op->mat, mat.data(), mat.size(), s);
@@ -414,7 +433,9 @@ void build_fused(rfhip_op *op, const rfhip_op_desc &d) {
   a.nbr_node = op->nbr_node.as<int>();
   a.nbase = nbase.empty() ? nullptr : op->nbase.as<int>();
   a.clane = has_clane ? op->clane.as<double>() : nullptr;
-  a.variant = default_variant(op->order, op->form);
+  a.quad = has_quad ? op->quad.as<double>() : nullptr;
+  a.quad_nodes = has_quad ? op->quad_nodes.p : nullptr;
+  a.variant = default_variant(op->order, op->form, a);
 }
 
 // ---- vectors at the boundary ---------------------------------------------

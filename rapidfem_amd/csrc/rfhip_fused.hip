@@ -2241,7 +2241,9 @@ inline int64_t resident_blocks(const void *kernel) { return resident_blocks_nt(k
 //         block-wide barriers in the group loop, unrolled by 2 / 4;
 //   8     k_clane: one lane per (element, field component), D_k and LIFT
 //         as wave-uniform scalar operands, the zeros of D_k skipped
-//         (operators whose reference element matches ElemTab).
+//         (operators whose reference element matches ElemTab);
+//   9     k_quad (rfhip_quad.hip): FP64 MFMA volume and LIFT, eight elements
+//         per wave (ElemTab's element; state under 2^32 bytes in FP64).
 // Variants 3 to 7 read the neighbour-trace table (built for conforming
 // meshes); variant 3 needs Np <= 20 (variant_available).
 
@@ -2533,6 +2535,7 @@ bool variant_available(int order, int form, int variant, const StageArgs &a) {
   const int np = (order + 1) * (order + 2) * (order + 3) / 6;
   if (form_vmf(form)) return variant >= 0 && variant < kStageVariantsBf16 && a.nbase != nullptr && order >= 2 && order <= 4;
   if (variant < 0 || variant >= kStageVariants) return false;
+  if (variant == kQuadVariant) return a.quad != nullptr;
   if (variant == 8) return a.clane != nullptr;
   if (variant == 3) return a.nbase != nullptr && np <= 20;
   if (variant >= 4) return a.nbase != nullptr;
@@ -2609,6 +2612,8 @@ bool clane_pack_np(const int *face_nodes, const double *const D[3], const double
 bool kcl_stage_fusable(int form, const StageArgs &a) { return !form_vmf(form) && a.nbase != nullptr; }
 
 int64_t kcl_stage_slots(int order, const StageArgs &a, bool r64) {
+  if (a.variant == kQuadVariant && a.quad)
+    return quad_kcl_slots((order + 1) * (order + 2) * (order + 3) / 6, r64, a.n_elem);
   switch ((order + 1) * (order + 2) * (order + 3) / 6) {
     case 4: return kcl_grid<4>(a, r64) * (kFusedWG / 64);
     case 10: return kcl_grid<10>(a, r64) * (kFusedWG / 64);
@@ -2621,6 +2626,10 @@ int64_t kcl_stage_slots(int order, const StageArgs &a, bool r64) {
 void launch_kcl_stage(int order, const StageArgs &a, bool r64, hipStream_t s) {
   RF_REQUIRE(a.nbase != nullptr, "the fused KCL stage needs the neighbour-trace table");
   RF_REQUIRE(!a.klast || a.kpart != nullptr, "the last KCL stage needs the error partials");
+  if (a.variant == kQuadVariant && a.quad) {
+    launch_quad((order + 1) * (order + 2) * (order + 3) / 6, r64 ? 4 : 3, a, s);
+    return;
+  }
   switch ((order + 1) * (order + 2) * (order + 3) / 6) {
     case 4: kcl_np<4>(a, r64, s); break;
     case 10: kcl_np<10>(a, r64, s); break;
@@ -2650,6 +2659,10 @@ void launch_stage(int order, int form, int epi, const StageArgs &a, hipStream_t 
       vmf_dispatch<false, 0>(np, vmf, variant, a, s);
     else
       vmf_dispatch<true, 2>(np, vmf, variant, a, s);
+    return;
+  }
+  if (variant == kQuadVariant && a.quad) {
+    launch_quad(np, epi == 0 ? 0 : form_compressed(form) ? 2 : 1, a, s);
     return;
   }
   if (epi == 0)

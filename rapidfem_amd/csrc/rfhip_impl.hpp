@@ -155,6 +155,8 @@ struct StageArgs {
   const int *nbr_node;    // [(f*4 + nlf)*6 + orientation][Nfp] -> neighbour volume node
   const int *nbase;       // [e*4Nfp + fm]: AoS index of the neighbour trace, or the (negative) face code
   const double *clane;    // nonzeros of D_k then LIFT, in k_clane's order (clane_pack), or null
+  const double *quad;     // A fragments of D_k's nonzero 4x4 blocks then LIFT, in k_quad's order (quad_pack), or null
+  const void *quad_nodes; // 100 rows of 16 node numbers (bytes): (f*4 + nlf)*6 + orientation, then 96 + f the own face
   const void *yin;        // double, or float hi (compressed)
   const void *yin_lo;     // bf16 lo (compressed) or null
   void *yout, *yout_lo;
@@ -199,7 +201,7 @@ struct rfhip_op {
   // device operator data
   rfhip::DevBuf dr, ds, dt, lift, face_nodes, jinv, inv_eps, inv_mu, sig_eps, sig_mu, normal, fscale, nbr,
       nbr_lf, port, perm;
-  rfhip::DevBuf dT, liftc, lfrag, afrag7, afragb, clane, jinv64, fcode, mat, mat_tab, nbr_node, nbase;
+  rfhip::DevBuf dT, liftc, lfrag, afrag7, afragb, clane, quad, quad_nodes, jinv64, fcode, mat, mat_tab, nbr_node, nbase;
   int64_t n_vec = 0;  // length of device vectors (n_dof)
   // Debye dispersive block: slot -> element and (a, g, 1/eps_inf); the P
   // block follows the 6 Np K values of [E,H] in every state vector
@@ -273,7 +275,8 @@ void launch_add_vec(const rfhip_op *op, void *k, const void *src, double g, hipS
 // Fused forms: epi 0 = apply (dy), 1 = LSERK stage (FP64 or compressed
 // registers by form). Stage-kernel variants 0 .. kStageVariants-1 (the
 // precision forms: 0 .. kStageVariantsBf16-1).
-constexpr int kStageVariants = 9;
+constexpr int kStageVariants = 10;
+constexpr int kQuadVariant = 9;  // k_quad (rfhip_quad.hip)
 constexpr int kStageVariantsBf16 = 2;
 void launch_stage(int order, int form, int epi, const StageArgs &a, hipStream_t s);
 // Whether stage-kernel variant `variant` runs as itself on this operator's
@@ -296,6 +299,14 @@ void launch_kcl_stage(int order, const StageArgs &a, bool r64, hipStream_t s);
 // ((face, node, face node) order). False when the operator's face nodes or
 // the zeros of its D_k differ from the compiled equispaced tables.
 bool clane_pack(int np, const int *face_nodes, const double *const D[3], const double *lift, std::vector<double> &out);
+// k_quad (stage-kernel variant 9, rfhip_quad.hip): its fragment table from
+// D_k and LIFT of the compiled equispaced element (clane_pack holds), the
+// launch (epi 0 apply, 1 / 2 LSERK4 stage with FP64 / compressed registers,
+// 3 / 4 KCL stage with compressed / FP64 registers) and the number of partial
+// sums its last KCL stage leaves in a.kpart.
+void quad_pack(int np, const double *const D[3], const double *lift, std::vector<double> &out);
+void launch_quad(int np, int epi, const StageArgs &a, hipStream_t s);
+int64_t quad_kcl_slots(int np, bool r64, int64_t n_elem);
 // Debye block after an applied derivative (dy = A y; f32: plain FP32 form),
 // with the drive of the P rows, and after a fused LSERK4 stage
 // (rfhip_debye.hip). No-ops without Debye elements.

@@ -1,0 +1,972 @@
+// FP64 stage kernel on v_mfma_f64_4x4x4_4b (stage-kernel variant 9).
+//
+// One wave owns a group of 8 elements and holds it as 16 columns: column
+// 2 el + fld is field fld (0 = E, 1 = H) of element el. In the layout of
+// v_mfma_f64_4x4x4_4b lane l = 16 q + c has column c of row q of B and of the
+// result, so
+//  * volume: the Np nodes are dealt into groups of four, node(g, q); lane q
+//    of a column reads its three field components at node(b, q) from LDS and
+//    they are the B operands of block column b as they stand. The product for
+//    output group a, derivative k hands lane q the reference derivative at its
+//    own node(a, q): J^-1, the curl and the accumulators never leave the lane;
+//    the curl of one field is the other field's right-hand side and moves to
+//    the neighbouring lane (l ^ 1) with a DPP quad permute.
+//  * flux: lane q of a column owns local face q: one face code, one normal
+//    and the face's Nfp nodes one after the other. The three flux components
+//    of face node s are the B operands of LIFT's columns {f Nfp + s}, again as
+//    they stand; the partner field's jump comes over the same DPP permute.
+//    Neighbour nodes come from the face code and a 16-byte row of packed node
+//    numbers in LDS (no per-face-node table is read from HBM).
+//  * D_k is sparse on equispaced nodes: 4x4 blocks of D_k that are zero are
+//    left out at compile time, and the node groups below are the ones an
+//    annealed search found to leave the fewest: 20 of 27, 49 of 75 and 138 of
+//    243 blocks at N = 2, 3, 4 (24 % to 43 % of the volume products).
+//  * state in and stage update out are linear over the group (16-byte or
+//    8 + 4 byte loads and stores per lane, no lane idle): y goes to LDS as FP64,
+//    and the right-hand side comes back through the same LDS.
+// On MI355X v_mfma_f64_4x4x4_4b runs at the vector unit's FP64 rate (70
+// TFLOP/s measured, v_mfma_f64_16x16x4 48) and shares its cycles with vector
+// instructions, so what it saves over FMAs is operand traffic (D and LIFT as
+// one LDS read per 4 x 4 x 16 products instead of one per lane and node) and
+// idle lanes (29 of 64 with one lane per node at N = 4).
+//
+// What bounds it (LSERK4 stage, FP64 registers, 324,000 tets at N = 3, 290 us
+// against 416 for the variant before it): the memory side. Leaving out all
+// products changes nothing, streaming the state and p alone takes 245 us (5.3
+// TB/s), the neighbour traces, 10 M line requests to L2, the rest. At N = 4
+// (384,000 tets, 687 us against 1232) products and vector instructions fill
+// about 70 % of the issue cycles.
+#include <algorithm>
+#include <map>
+#include <mutex>
+#include <tuple>
+#include <type_traits>
+#include <vector>
+
+#include "rfhip_elem_tables.hpp"
+#include "rfhip_impl.hpp"
+#include "rfhip_regs.hpp"
+
+namespace rfhip {
+namespace {
+
+constexpr int kQuadEl = 8;  // elements per wave
+
+// Node groups: NODE[g][q] is the node of lane q in group g (Np: none). NWB:
+// waves per block (they share the tables in LDS). TW: neighbour traces
+// requested ahead of the previous group's stores. RING: fragment pairs in
+// registers. LATE: the state is read at the group's start and the update's
+// registers after LIFT instead of one phase earlier, for want of registers: at
+// N = 4 the early reads spill 34 to 100 of them, and since a reload waits in
+// order behind the stores that costs more (929 us against 703 per FP64 stage
+// of 384,000 tets). TW and RING are the fastest of 2 to 10 and 2 to 5.
+template <int NP>
+struct QuadTab;
+template <>
+struct QuadTab<4> {
+  static constexpr int NG = 1, NWB = 4, TW = 3, RING = 4;
+  static constexpr bool LATE = false;
+  static constexpr int NODE[NG][4] = {{0, 1, 2, 3}};
+};
+template <>
+struct QuadTab<10> {
+  static constexpr int NG = 3, NWB = 4, TW = 6, RING = 4;
+  static constexpr bool LATE = false;
+  static constexpr int NODE[NG][4] = {{4, 1, 7, 2}, {10, 10, 9, 8}, {3, 6, 0, 5}};
+};
+template <>
+struct QuadTab<20> {
+  static constexpr int NG = 5, NWB = 4, TW = 4, RING = 4;
+  static constexpr bool LATE = false;
+  static constexpr int NODE[NG][4] = {{6, 3, 12, 2}, {17, 18, 19, 16}, {5, 0, 4, 1}, {14, 11, 10, 13}, {15, 9, 8, 7}};
+};
+template <>
+struct QuadTab<35> {
+  static constexpr int NG = 9, NWB = 8, TW = 2, RING = 3;
+  static constexpr bool LATE = true;
+  static constexpr int NODE[NG][4] = {{7, 11, 21, 8},  {30, 33, 28, 29}, {19, 20, 23, 22}, {9, 6, 10, 5}, {16, 15, 0, 1},
+                                      {24, 12, 13, 14}, {4, 17, 3, 2},   {25, 18, 26, 27}, {32, 35, 31, 34}};
+};
+
+// Whether block (a, b) of D_k has a nonzero.
+template <int NP>
+constexpr bool quad_nz(int k, int a, int b) {
+  for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < 4; ++j) {
+      const int r = QuadTab<NP>::NODE[a][i], c = QuadTab<NP>::NODE[b][j];
+      if (r < NP && c < NP && ((ElemTab<NP>::DM[k][r] >> c) & 1ull)) return true;
+    }
+  return false;
+}
+// Blocks before (a, b, k) in the order the kernel reads them (k fastest);
+// quad_at<NP>(NG, 0, 0) counts them all and LIFT's fragments start there.
+template <int NP>
+constexpr int quad_at(int a_end, int b_end, int k_end) {
+  int s = 0;
+  for (int a = 0; a < QuadTab<NP>::NG; ++a)
+    for (int b = 0; b < QuadTab<NP>::NG; ++b)
+      for (int k = 0; k < 3; ++k) {
+        if (a > a_end || (a == a_end && (b > b_end || (b == b_end && k >= k_end)))) return s;
+        s += quad_nz<NP>(k, a, b) ? 1 : 0;
+      }
+  return s;
+}
+// Steps of the volume: the blocks (a, b), a-major, where any D_k has a nonzero.
+template <int NP>
+constexpr int quad_steps() {
+  int n = 0;
+  for (int ab = 0; ab < QuadTab<NP>::NG * QuadTab<NP>::NG; ++ab)
+    n += quad_nz<NP>(0, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG) || quad_nz<NP>(1, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG) ||
+         quad_nz<NP>(2, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG);
+  return n;
+}
+template <int NP>
+constexpr int quad_step(int st) {
+  constexpr int NG = QuadTab<NP>::NG;
+  for (int ab = 0; ab < NG * NG; ++ab)
+    if (quad_nz<NP>(0, ab / NG, ab % NG) || quad_nz<NP>(1, ab / NG, ab % NG) || quad_nz<NP>(2, ab / NG, ab % NG))
+      if (st-- == 0) return ab;
+  return -1;
+}
+template <int NP>
+struct QuadSize {
+  static constexpr int NV = quad_at<NP>(QuadTab<NP>::NG, 0, 0);
+  static constexpr int NL = ElemTab<NP>::NFP * QuadTab<NP>::NG;
+  static constexpr int NF = NV + NL;  // A fragments of 16 doubles
+};
+
+template <int B, int E, class F>
+__device__ __forceinline__ void unroll(F &&f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    unroll<B + 1, E>(f);
+  }
+}
+
+// The value of the other field's lane of the same element (lane l ^ 1).
+__device__ __forceinline__ double other_field(double v) {
+  const int2 w = __builtin_bit_cast(int2, v);
+  const int lo = __builtin_amdgcn_mov_dpp(w.x, 0xB1, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(w.y, 0xB1, 0xF, 0xF, true);
+  return __builtin_bit_cast(double, make_int2(lo, hi));
+}
+
+// Two floats to bf16 (round to nearest even), a in the low half. As an
+// instruction of its own: from (float)double operands the compiler forms an
+// f64 -> bf16 conversion of six vector instructions and a branch per value.
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  uint32_t r;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double c_f64(float h, uint32_t lo_bits) { return (double)h + (double)__uint_as_float(lo_bits); }
+
+struct F3 {
+  float x, y, z;
+};
+struct D3 {
+  double x, y, z;
+};
+struct U2 {
+  uint32_t x, y;
+};
+
+// Three values of one field at one node as stored: f32 + the 8 bytes that
+// hold its bf16 parts, or f64.
+template <bool CIN>
+struct Trace;
+template <>
+struct Trace<true> {
+  F3 h;
+  U2 l;
+};
+template <>
+struct Trace<false> {
+  D3 d;
+};
+
+// VW consecutive values of a linear register as stored.
+template <bool CIN, int VW>
+struct Lin;
+template <>
+struct Lin<true, 4> {
+  float4 h;
+  uint2 l;
+};
+template <>
+struct Lin<true, 2> {
+  float2 h;
+  uint32_t l;
+};
+template <int VW>
+struct Lin<false, VW> {
+  double2 d[VW / 2];
+};
+
+template <class T>
+__device__ __forceinline__ T ld(const void *p, uint32_t byte) {
+  T v;
+  __builtin_memcpy(&v, static_cast<const char *>(p) + byte, sizeof(T));
+  return v;
+}
+template <class T>
+__device__ __forceinline__ T ld_al(const void *p, uint32_t byte) {
+  return *reinterpret_cast<const T *>(static_cast<const char *>(p) + byte);
+}
+// Streamed accesses: the update's registers and every store are touched once
+// per launch and are kept from displacing the state that neighbours gather.
+template <class T>
+__device__ __forceinline__ T ld_nt(const void *p, uint32_t byte) {
+  typedef unsigned W __attribute__((ext_vector_type(sizeof(T) / 4)));
+  return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const W *>(static_cast<const char *>(p) + byte)));
+}
+template <class T>
+__device__ __forceinline__ void st_al(void *p, uint32_t byte, T v) {
+  typedef unsigned W __attribute__((ext_vector_type(sizeof(T) / 4)));
+  __builtin_nontemporal_store(__builtin_bit_cast(W, v), reinterpret_cast<W *>(static_cast<char *>(p) + byte));
+}
+
+template <bool CIN, int VW, bool NT = false>
+__device__ __forceinline__ Lin<CIN, VW> load_lin(const void *hi, const void *lo, uint32_t i) {
+  auto get = [](auto z, const void *p, uint32_t byte) {
+    using V = decltype(z);
+    if constexpr (NT) return ld_nt<V>(p, byte);
+    else return ld_al<V>(p, byte);
+  };
+  Lin<CIN, VW> r;
+  if constexpr (CIN && VW == 4) {
+    r.h = get(float4{}, hi, 4 * i);
+    r.l = get(uint2{}, lo, 2 * i);
+  } else if constexpr (CIN) {
+    r.h = get(float2{}, hi, 4 * i);
+    r.l = get(uint32_t{}, lo, 2 * i);
+  } else {
+#pragma unroll
+    for (int v = 0; v < VW / 2; ++v) r.d[v] = get(double2{}, hi, 8 * i + 16 * v);
+  }
+  return r;
+}
+template <bool CIN, int VW>
+__device__ __forceinline__ void lin_f64(const Lin<CIN, VW> &r, double *v) {
+  if constexpr (CIN && VW == 4) {
+    v[0] = c_f64(r.h.x, r.l.x << 16);
+    v[1] = c_f64(r.h.y, r.l.x & 0xFFFF0000u);
+    v[2] = c_f64(r.h.z, r.l.y << 16);
+    v[3] = c_f64(r.h.w, r.l.y & 0xFFFF0000u);
+  } else if constexpr (CIN) {
+    v[0] = c_f64(r.h.x, r.l << 16);
+    v[1] = c_f64(r.h.y, r.l & 0xFFFF0000u);
+  } else {
+#pragma unroll
+    for (int q = 0; q < VW / 2; ++q) {
+      v[2 * q] = r.d[q].x;
+      v[2 * q + 1] = r.d[q].y;
+    }
+  }
+}
+// VW FP64 values stored as f32 hi + bf16 lo.
+template <int VW>
+__device__ __forceinline__ void store_c(void *hi, void *lo, uint32_t i, const double *v) {
+  float h[VW], r[VW];
+#pragma unroll
+  for (int q = 0; q < VW; ++q) {
+    h[q] = (float)v[q];
+    r[q] = (float)(v[q] - (double)h[q]);
+  }
+  if constexpr (VW == 4) {
+    st_al(hi, 4 * i, make_float4(h[0], h[1], h[2], h[3]));
+    st_al(lo, 2 * i, make_uint2(bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3])));
+  } else {
+    st_al(hi, 4 * i, make_float2(h[0], h[1]));
+    st_al(lo, 2 * i, bf16_pair(r[0], r[1]));
+  }
+}
+template <int VW>
+__device__ __forceinline__ void store_d(void *p, uint32_t i, const double *v) {
+#pragma unroll
+  for (int q = 0; q < VW / 2; ++q) st_al(p, 8 * i + 16 * q, make_double2(v[2 * q], v[2 * q + 1]));
+}
+template <int VW>
+__device__ __forceinline__ void store_f(void *p, uint32_t i, const float *v) {
+  if constexpr (VW == 4)
+    st_al(p, 4 * i, make_float4(v[0], v[1], v[2], v[3]));
+  else
+    st_al(p, 4 * i, make_float2(v[0], v[1]));
+}
+template <int VW>
+struct Flt {
+  float v[VW];
+};
+template <int VW>
+__device__ __forceinline__ Flt<VW> load_f(const void *p, uint32_t i) {
+  if constexpr (VW == 4) {
+    const float4 t = ld_nt<float4>(p, 4 * i);
+    return {{t.x, t.y, t.z, t.w}};
+  } else {
+    const float2 t = ld_nt<float2>(p, 4 * i);
+    return {{t.x, t.y}};
+  }
+}
+
+// The linear registers an epilogue reads besides the state: p (LSERK4) or y
+// and err (KCL).
+template <int EPI, int VW>
+struct Upd {};
+template <int VW>
+struct Upd<1, VW> {
+  Lin<false, VW> p;
+  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) { p = load_lin<false, VW, true>(io.p, nullptr, i); }
+};
+template <int VW>
+struct Upd<2, VW> {
+  Flt<VW> p;
+  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) { p = load_f<VW>(io.p, i); }
+};
+template <int VW>
+struct Upd<3, VW> {
+  Lin<true, VW> y;
+  Flt<VW> e;
+  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) {
+    y = load_lin<true, VW, true>(io.ky, io.ky_lo, i);
+    e = load_f<VW>(io.kerr, i);
+  }
+};
+template <int VW>
+struct Upd<4, VW> {
+  Lin<false, VW> y, e;
+  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) {
+    y = load_lin<false, VW, true>(io.kyd, nullptr, i);
+    e = load_lin<false, VW, true>(io.kerrd, nullptr, i);
+  }
+};
+
+__device__ __forceinline__ int64_t quad_block() {
+  const unsigned nb = gridDim.x;
+  return (nb & 7u) == 0 ? (int64_t)(blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
+}
+
+// Waves per SIMD the registers are fitted to: the most that leave no spills
+// (N = 2: 300 us at 3 waves, 342 at 2 with compressed registers; 427 at 3 with
+// 13 spilled, 350 at 2, with FP64 ones; N = 3 at 3 waves spills 48 to 100).
+template <int NP, int EPI>
+struct QuadWaves {
+  static constexpr int v = NP == 4 ? 4 : NP == 10 && (EPI == 0 || EPI == 2) ? 3 : 2;
+};
+
+// EPI as in the other stage kernels: 0 apply, 1 LSERK4 stage with FP64
+// registers, 2 with compressed ones, 3 / 4 KCL stage with compressed / FP64
+// registers. CIN: the input state is f32 + bf16. nw: the waves of a block that
+// take groups (all of them load the tables).
+template <int NP, bool CIN, int EPI>
+__global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_waves_per_eu(QuadWaves<NP, EPI>::v))) k_quad(StageArgs io, int nw) {
+  using T = QuadTab<NP>;
+  using Z = QuadSize<NP>;
+  constexpr int NG = T::NG, NT = T::NWB * 64, NFP = ElemTab<NP>::NFP;
+  constexpr int SE = 6 * NP;             // values per element
+  constexpr int SW = kQuadEl * SE;       // values per group
+  // Element stride in LDS, = 4 mod 8 in 8-byte banks: with the nodes of lanes
+  // q = 0, 1 (and 2, 3) of a group of different parity, the 32 lanes of a half
+  // wave then read their 8-byte values from different banks.
+  constexpr int SP = SE + (12 - SE % 8) % 8;
+  constexpr int SZ = kQuadEl * SP;
+  constexpr int VW = CIN && SE % 4 == 0 ? 4 : 2;
+  constexpr int IT = (SW / VW + 63) / 64;
+  constexpr int NFR = (Z::NF + 1) / 2;   // fragment pairs
+  __shared__ __align__(16) double sA[NFR * 32];
+  __shared__ __align__(16) uint4 snode[100];
+  __shared__ int splace[4 * NG];
+  __shared__ __align__(16) double su_b[T::NWB][SZ + 8];  // + zeros the padding nodes read, + a place for what they write
+  for (int t = threadIdx.x; t < NFR * 16; t += NT) reinterpret_cast<double2 *>(sA)[t] = reinterpret_cast<const double2 *>(io.quad)[t];
+  for (int t = threadIdx.x; t < 100; t += NT) snode[t] = reinterpret_cast<const uint4 *>(io.quad_nodes)[t];
+  if ((int)threadIdx.x < 4 * NG) splace[threadIdx.x] = 6 * T::NODE[threadIdx.x / 4][threadIdx.x % 4];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  double *su = su_b[wave];
+  double2 *su2 = reinterpret_cast<double2 *>(su);
+  auto at = [](int i) { return i + (i / SE) * (SP - SE); };  // LDS place of value i of the group
+  const int64_t ngroups = (io.n_elem + kQuadEl - 1) / kQuadEl;
+  const int64_t gw0 = quad_block() * nw + wave, gws = (int64_t)gridDim.x * nw;
+  __syncthreads();  // the only block-wide barrier: the tables are in LDS
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  if (lane < 4) su[SZ + lane] = 0.0;
+  const int64_t wslot = (int64_t)blockIdx.x * nw + wave;
+  double wsum = 0.0;
+  if (wave >= nw || gw0 >= ngroups) {
+    if constexpr (EPI == 3 || EPI == 4)
+      if (wave < nw && io.klast && (threadIdx.x & 63) == 0) io.kpart[wslot] = 0.0;
+    return;
+  }
+  const int q = lane >> 4, fld = lane & 1, el = (lane >> 1) & 7;
+  // A operand: lane 16 kk + 4 b + i reads entry (kk, i) of a fragment for every b; pair t: fr[16 t]
+  const double2 *fr = reinterpret_cast<const double2 *>(sA) + (4 * q + (lane & 3));
+  // LDS index of this lane's three values at node(g, q), from a table where
+  // they are used (held for the whole group they would cost NG registers).
+  auto places = [&](int (&un)[NG]) {
+    int t = q;
+    asm volatile("" : "+v"(t));
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const int n = splace[4 * g + t];
+      un[g] = n < SE ? el * SP + n + 3 * fld : SZ;
+    }
+  };
+
+  // Every load a group needs before its LIFT is issued ahead of the stores of
+  // the group before it: its state (nx), J^-1, materials and first neighbour
+  // traces. Vector memory operations retire in order, so a load behind those
+  // stores would be waited for together with them. Face codes and material
+  // indices, which those loads depend on, run two groups ahead.
+  // All loads are unconditional, with clamped indices.
+  Lin<CIN, VW> nx[IT];
+  auto read_state = [&](int64_t g, int ln) {
+    const int64_t rg = io.n_elem - g * kQuadEl;
+    const int ng = rg < kQuadEl ? (int)rg : kQuadEl;
+    const uint32_t gb = (uint32_t)g * SW, last = gb + (uint32_t)(ng * SE - VW);
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const uint32_t i = gb + (uint32_t)(ln + 64 * k) * VW;
+      nx[k] = load_lin<CIN, VW>(io.yin, io.yin_lo, i < last ? i : last);
+    }
+  };
+  auto elem_of = [&](int64_t g) {
+    const int64_t rg = io.n_elem - g * kQuadEl;
+    const int ng = rg < kQuadEl ? (int)rg : kQuadEl;
+    return (uint32_t)g * kQuadEl + (uint32_t)(el < ng ? el : ng - 1);
+  };
+  auto node_of = [](const uint4 &r, int s) {
+    const uint32_t w = s < 4 ? r.x : s < 8 ? r.y : s < 12 ? r.z : r.w;
+    return (w >> (8 * (s & 3))) & 0xFFu;
+  };
+  // A window of TW neighbour traces is in flight: each slot, once used, takes
+  // the trace TW face nodes on. A wall or port face reads its own trace.
+  constexpr int TW = NFP < T::TW ? NFP : T::TW;
+  constexpr bool ROLL = T::LATE;
+  constexpr int NTR = ROLL ? TW : NFP;
+  Trace<CIN> tr[NTR];
+  uint4 nrow;
+  uint32_t tbh, tbl;
+  auto load_trace = [&](int s) {
+    const uint32_t n = node_of(nrow, s);
+    if constexpr (CIN) {
+      tr[s % NTR].h = ld<F3>(io.yin, tbh + 24 * n);
+      tr[s % NTR].l = ld<U2>(io.yin_lo, tbl + 12 * n);
+    } else {
+      tr[s % NTR].d = ld<D3>(io.yin, tbh + 48 * n);
+    }
+  };
+  struct J9 {
+    double v[9];
+  };
+  J9 jr;
+  auto read_geom = [&](int64_t g, int code) {
+    const uint32_t e = elem_of(g);
+    const int bnd = code >> 31;  // all ones on a wall or port face; masks, not a lane-divergent branch
+    const uint32_t ne = (uint32_t)(((code >> 5) & ~bnd) | ((int)e & bnd));
+    nrow = snode[((24 * q + 6 * ((code >> 3) & 3) + (code & 7)) & ~bnd) | ((96 + q) & bnd)];
+    tbh = ne * (uint32_t)(SE * (CIN ? 4 : 8)) + (CIN ? 12 : 24) * fld;
+    tbl = ne * (uint32_t)(2 * SE) + 4 * fld;
+    jr = ld<J9>(io.jinv, 72 * e);
+#pragma unroll
+    for (int s = 0; s < TW; ++s) load_trace(s);
+  };
+  auto next_of = [&](int64_t g) { return g + gws < ngroups ? g + gws : g; };
+  int code, mat, ncode, nmat;
+  {
+    const uint32_t e0 = elem_of(gw0), e1 = elem_of(next_of(gw0));
+    code = io.fcode[4 * e0 + q];
+    mat = io.mat[e0];
+    ncode = io.fcode[4 * e1 + q];
+    nmat = io.mat[e1];
+    read_state(gw0, lane);
+    read_geom(gw0, code);
+  }
+
+#pragma unroll 1
+  for (int64_t grp = gw0; grp < ngroups; grp += gws) {
+    const int64_t rem = io.n_elem - grp * kQuadEl;
+    const int nel = rem < kQuadEl ? (int)rem : kQuadEl;
+    const uint32_t gb = (uint32_t)grp * SW;
+    // An opaque copy of the lane id, so the places of this lane's linear
+    // values are formed where they are used and not held in registers.
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+
+    if constexpr (T::LATE) read_state(grp, ln);
+    // the group's state to LDS
+#pragma unroll
+    for (int k = 0; k < IT; ++k) {
+      const int i = (ln + 64 * k) * VW;
+      const int to = (SW / VW) % 64 == 0 || k < IT - 1 || i < SW ? at(i) : SZ + 4;
+      double v[VW];
+      lin_f64<CIN, VW>(nx[k], v);
+#pragma unroll
+      for (int c = 0; c < VW / 2; ++c) su2[to / 2 + c] = make_double2(v[2 * c], v[2 * c + 1]);
+    }
+    if constexpr (!ROLL) {
+#pragma unroll
+      for (int s = TW; s < NFP; ++s) load_trace(s);
+    }
+    double ji[9];
+    {
+      const double sg = fld ? 1.0 : -1.0;  // the curl of E enters dH/dt with a minus, and so does n x [H] dE/dt
+#pragma unroll
+      for (int c = 0; c < 9; ++c) ji[c] = sg * jr.v[c];
+    }
+    wave_sync();
+
+    // Fragment pairs are read kRing - 1 pairs ahead of their products, in an
+    // order the scheduler may not change: left to it, every read is issued
+    // right before its first product and waited for there.
+    constexpr int kRing = T::RING;
+    double2 ring[kRing];
+#pragma unroll
+    for (int t = 0; t < kRing - 1; ++t) ring[t] = fr[16 * t];
+    auto frag = [&](auto fc) {
+      constexpr int t = fc / 2, ahead = t + kRing - 1;
+      if constexpr (fc % 2 == 0) {
+        if constexpr (ahead < NFR) ring[ahead % kRing] = fr[16 * ahead];
+        if constexpr (fc < Z::NV) __builtin_amdgcn_sched_barrier(0);
+      }
+      return fc % 2 ? ring[t % kRing].y : ring[t % kRing].x;
+    };
+
+    // Volume: reference derivatives of this lane's field at its nodes, J^-1,
+    // the curl, and over to the other field. The state operands come from LDS,
+    // one block ahead of their products (held in registers for the whole
+    // volume they would cost 6 Np / 4 of them).
+    double acc[NG][3];
+    double ub[2][3];
+    int un[NG];
+    places(un);
+    auto operand = [&](auto bc) {
+      constexpr int st = bc;  // step: block (a, b) = (quad_step / NG, quad_step % NG)
+      constexpr int ab = quad_step<NP>(st);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) ub[st & 1][c] = su[un[ab % NG] + c];
+    };
+    constexpr int NST = quad_steps<NP>();
+    operand(std::integral_constant<int, 0>{});
+    double r[3][3];
+    unroll<0, NST>([&](auto sc) {
+      constexpr int st = sc, ab = quad_step<NP>(st), a = ab / NG, b = ab % NG;
+      if constexpr (st == 0 || quad_step<NP>(st - 1) / NG != a) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+          for (int c = 0; c < 3; ++c) r[k][c] = 0.0;
+      }
+      if constexpr (st + 1 < NST) operand(std::integral_constant<int, st + 1>{});
+      unroll<0, 3>([&](auto kc) {
+        constexpr int k = kc;
+        if constexpr (quad_nz<NP>(k, a, b)) {
+          const double f = frag(std::integral_constant<int, quad_at<NP>(a, b, k)>{});
+#pragma unroll
+          for (int c = 0; c < 3; ++c) r[k][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(f, ub[st & 1][c], r[k][c], 0, 0, 0);
+        }
+      });
+      if constexpr (st + 1 == NST || quad_step<NP>(st + 1) / NG != a) {
+        auto pd = [&](int p, int c) { return ji[p] * r[0][c] + ji[3 + p] * r[1][c] + ji[6 + p] * r[2][c]; };
+        acc[a][0] = other_field(pd(1, 2) - pd(2, 1));
+        acc[a][1] = other_field(pd(2, 0) - pd(0, 2));
+        acc[a][2] = other_field(pd(0, 1) - pd(1, 0));
+      }
+    });
+
+    // The next group's state and the registers the update reads, linear like
+    // the state; requested here so the flux and LIFT cover their latency (the
+    // volume's operands are free).
+    __builtin_amdgcn_sched_barrier(0);
+    const int64_t grp1 = next_of(grp);
+    if constexpr (!T::LATE) read_state(grp1, ln);
+    int nncode, nnmat;
+    {
+      const uint32_t e2 = elem_of(next_of(grp1));
+      nncode = io.fcode[4 * e2 + q];
+      nnmat = io.mat[e2];
+    }
+    Upd<EPI, VW> up[EPI == 0 ? 1 : IT];
+    auto read_registers = [&] {
+      if constexpr (EPI != 0) {
+        const uint32_t last = gb + (uint32_t)(nel * SE - VW);
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+          const uint32_t i = gb + (uint32_t)(ln + 64 * k) * VW;
+          up[k].load(io, i < last ? i : last);
+        }
+      }
+    };
+    if constexpr (!T::LATE) read_registers();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+
+    // Face geometry: m = -+ 0.5 g = -+ cf n of face q (sign as ji), cf = |m|.
+    double m[3];
+    // m = a row of J^-1 or their sum: weights 0, +-1/2 per lane, without branches
+    const double wr0 = q == 1 ? -0.5 : q == 3 ? 0.5 : 0.0, wr1 = q == 2 ? -0.5 : q == 3 ? 0.5 : 0.0,
+                 wr2 = q == 0 ? -0.5 : q == 3 ? 0.5 : 0.0;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) m[x] = wr0 * ji[x] + wr1 * ji[3 + x] + wr2 * ji[6 + x];
+    const double ss = m[0] * m[0] + m[1] * m[1] + m[2] * m[2], hs = 0.5 * ss;
+    double ic = __builtin_amdgcn_rsq(ss);  // 1 / cf, two Newton steps as in face_geom
+    ic = ic * fma(-hs * ic, ic, 1.5);
+    ic = ic * fma(-hs * ic, ic, 1.5);
+    const double al = code < kCodePec ? 1.0 : io.alpha;
+    const double acf = al * (ss * ic), aic = al * ic;
+
+    // Flux and LIFT, one face node of every face at a time:
+    // F = m (m . j) a / cf - a cf j -+ m x j' (j: this field's jump, j' the
+    // other's), j = own + sx * neighbour. On a boundary face the trace read is
+    // the own one, and since F keeps the tangential part of either jump, the
+    // wall and port rules are this sign: PEC ([E] = 2 E_t, [H] = 2 H_n: j = 2 E
+    // and 0), port ([.] = the own trace). The flux of a node is formed while
+    // the products of the node before it run.
+    const double sx = code >= 0 ? -1.0 : code < kCodePec ? 0.0 : fld ? -1.0 : 1.0;
+    const double *const us = su + el * SP + 3 * fld;
+    int qo = 96 + q;
+    asm volatile("" : "+v"(qo));  // not a loop constant held in registers
+    const uint4 orow = snode[qo];
+    double ow[3];
+    auto own_trace = [&](int s) {
+      const double *p = us + node_of(orow, s) * 6;
+      ow[0] = p[0];
+      ow[1] = p[1];
+      ow[2] = p[2];
+    };
+    D3 minv, msig;
+    {
+      double F[2][3];
+      own_trace(0);
+      auto flux = [&](auto sc) {
+        constexpr int s = sc;
+        double j[3];
+        const Trace<CIN> x = tr[s % NTR];
+        if constexpr (CIN) {
+          const uint32_t sh = fld << 4;
+          const uint32_t l0 = __builtin_amdgcn_alignbit(x.l.y, x.l.x, sh), l1 = x.l.y >> sh;
+          j[0] = fma(sx, c_f64(x.h.x, l0 << 16), ow[0]);
+          j[1] = fma(sx, c_f64(x.h.y, l0 & 0xFFFF0000u), ow[1]);
+          j[2] = fma(sx, c_f64(x.h.z, l1 << 16), ow[2]);
+        } else {
+          j[0] = fma(sx, x.d.x, ow[0]);
+          j[1] = fma(sx, x.d.y, ow[1]);
+          j[2] = fma(sx, x.d.z, ow[2]);
+        }
+        if constexpr (ROLL && s + TW < NFP) load_trace(s + TW);
+        if constexpr (s + 1 < NFP) own_trace(s + 1);
+        double o[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) o[c] = other_field(j[c]);
+        const double t = aic * (m[0] * j[0] + m[1] * j[1] + m[2] * j[2]);
+        F[s & 1][0] = m[0] * t - acf * j[0] + (m[1] * o[2] - m[2] * o[1]);
+        F[s & 1][1] = m[1] * t - acf * j[1] + (m[2] * o[0] - m[0] * o[2]);
+        F[s & 1][2] = m[2] * t - acf * j[2] + (m[0] * o[1] - m[1] * o[0]);
+      };
+      flux(std::integral_constant<int, 0>{});
+      unroll<0, NFP>([&](auto sc) {
+        constexpr int s = sc;
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (s == (NFP > 3 ? NFP - 3 : 0)) {
+          minv = ld<D3>(io.mat_tab, 96 * (uint32_t)mat + 24 * fld);
+          msig = ld<D3>(io.mat_tab, 96 * (uint32_t)mat + 48 + 24 * fld);
+        }
+        if constexpr (s + 1 < NFP) flux(std::integral_constant<int, s + 1>{});
+        unroll<0, NG>([&](auto ac) {
+          constexpr int a = ac;
+          const double f = frag(std::integral_constant<int, Z::NV + s * NG + a>{});
+#pragma unroll
+          for (int c = 0; c < 3; ++c) acc[a][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(f, F[s & 1][c], acc[a][c], 0, 0, 0);
+        });
+      });
+    }
+
+    // Materials (rhs.rs:1443-1454), then the right-hand side to LDS in place
+    // of the state, which the update takes into registers first.
+    int up_at[NG];
+    places(up_at);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      acc[g][0] = minv.x * acc[g][0] - msig.x * su[up_at[g]];
+      acc[g][1] = minv.y * acc[g][1] - msig.y * su[up_at[g] + 1];
+      acc[g][2] = minv.z * acc[g][2] - msig.z * su[up_at[g] + 2];
+    }
+    // the next group's geometry and traces, ahead of this group's stores
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (T::LATE) read_registers();
+    code = ncode;
+    mat = nmat;
+    read_geom(grp1, code);
+    ncode = nncode;
+    nmat = nnmat;
+    __builtin_amdgcn_sched_barrier(0);
+    double yv[EPI == 1 || EPI == 2 ? IT : 1][VW];
+    if constexpr (EPI == 1 || EPI == 2) {
+#pragma unroll
+      for (int k = 0; k < IT; ++k) {
+        const int i = (ln + 64 * k) * VW, ic2 = i < SW ? i : 0;
+#pragma unroll
+        for (int c = 0; c < VW / 2; ++c) {
+          const double2 t = su2[at(ic2) / 2 + c];
+          yv[k][2 * c] = t.x;
+          yv[k][2 * c + 1] = t.y;
+        }
+      }
+    }
+    wave_sync();
+    unroll<0, NG>([&](auto gc) {
+      constexpr int g = gc;
+      constexpr bool pad = T::NODE[g][0] >= NP || T::NODE[g][1] >= NP || T::NODE[g][2] >= NP || T::NODE[g][3] >= NP;
+      const int to = pad && up_at[g] >= SZ ? SZ + 4 : up_at[g];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) su[to + c] = acc[g][c];
+    });
+    wave_sync();
+    const int nv = nel * SE;
+    auto update = [&](auto full) {
+      constexpr int CH = 4;  // iterations of right-hand sides in registers at a time
+#pragma unroll
+      for (int k0 = 0; k0 < IT; k0 += CH) {
+        double kr[CH][VW];
+#pragma unroll
+        for (int k = k0; k < (k0 + CH < IT ? k0 + CH : IT); ++k) {
+          const int i = (ln + 64 * k) * VW, ic2 = i < SW ? i : 0;
+#pragma unroll
+          for (int c = 0; c < VW / 2; ++c) {
+            const double2 t = su2[at(ic2) / 2 + c];
+            kr[k - k0][2 * c] = t.x;
+            kr[k - k0][2 * c + 1] = t.y;
+          }
+        }
+        if (io.src_kind == RFHIP_DRIVE_POINT) {
+          const int64_t off = io.src_dof - (int64_t)gb;
+#pragma unroll
+          for (int k = k0; k < (k0 + CH < IT ? k0 + CH : IT); ++k)
+#pragma unroll
+            for (int c = 0; c < VW; ++c)
+              if (off == (ln + 64 * k) * VW + c) kr[k - k0][c] += io.g;
+        } else if (io.src_kind == RFHIP_DRIVE_VECTOR) {
+#pragma unroll
+          for (int k = k0; k < (k0 + CH < IT ? k0 + CH : IT); ++k) {
+            const int i = (ln + 64 * k) * VW;
+            const double *sv = io.src_vec + gb + (i < nv ? i : 0);
+#pragma unroll
+            for (int c = 0; c < VW; ++c) kr[k - k0][c] += sv[c] * io.g;
+          }
+        }
+#pragma unroll
+        for (int k = k0; k < (k0 + CH < IT ? k0 + CH : IT); ++k) {
+          const int i = (ln + 64 * k) * VW;
+          if ((full && ((SW / VW) % 64 == 0 || k < IT - 1)) || i < nv) {
+            const double *kv = kr[k - k0];
+            const uint32_t gi = gb + (uint32_t)i;
+            if constexpr (EPI == 0) {
+              store_d<VW>(io.dy, gi, kv);
+            } else if constexpr (EPI == 1) {
+              double po[VW], pn[VW], yn[VW];
+              lin_f64<false, VW>(up[k].p, po);
+    #pragma unroll
+              for (int c = 0; c < VW; ++c) {
+                pn[c] = io.sa * po[c] + io.dt * kv[c];
+                yn[c] = yv[k][c] + io.sb * pn[c];
+              }
+              store_d<VW>(io.p, gi, pn);
+              store_d<VW>(io.yout, gi, yn);
+            } else if constexpr (EPI == 2) {
+              float pn[VW];
+              double yn[VW];
+    #pragma unroll
+              for (int c = 0; c < VW; ++c) {
+                pn[c] = (float)(io.sa * (double)up[k].p.v[c] + io.dt * kv[c]);
+                yn[c] = yv[k][c] + io.sb * (double)pn[c];
+              }
+              store_f<VW>(io.p, gi, pn);
+              store_c<VW>(io.yout, io.yout_lo, gi, yn);
+            } else if constexpr (EPI == 3) {
+              // the arithmetic of node_kcl (rfhip_fused.hip)
+              float en[VW];
+              double yn[VW], sn[VW], yo[VW], bo[VW];
+              if (io.klast) lin_f64<true, VW>(load_lin<true, VW>(io.kbak, io.kbak_lo, gi), bo);
+              lin_f64<true, VW>(up[k].y, yo);
+    #pragma unroll
+              for (int c = 0; c < VW; ++c) {
+                const double f = io.dt * kv[c];
+                yn[c] = yo[c] + io.kb * f;
+                const double er = io.kfirst ? io.kew * f : (double)up[k].e.v[c] + io.kew * f;
+                en[c] = (float)er;
+                sn[c] = io.klast ? yn[c] : yn[c] + io.kamb * f;
+                if (io.klast) wsum += werr_term(bo[c], yn[c], er, io.katol, io.krtol);
+              }
+              store_c<VW>(io.ky, io.ky_lo, gi, yn);
+              store_f<VW>(io.kerr, gi, en);
+              store_c<VW>(io.yout, io.yout_lo, gi, sn);
+              if (io.kfirst) {
+                st_al(io.kbak, 4 * gi, up[k].y.h);
+                st_al(io.kbak_lo, 2 * gi, up[k].y.l);
+              }
+            } else {
+              // the arithmetic of node_kcl64
+              double yo[VW], er[VW], bo[VW], sn[VW], yn[VW];
+              lin_f64<false, VW>(up[k].y, yo);
+              lin_f64<false, VW>(up[k].e, er);
+              if (io.klast) lin_f64<false, VW>(load_lin<false, VW>(io.kbakd, nullptr, gi), bo);
+    #pragma unroll
+              for (int c = 0; c < VW; ++c) {
+                const double f = io.dt * kv[c];
+                yn[c] = yo[c] + io.kb * f;
+                er[c] = io.kfirst ? io.kew * f : er[c] + io.kew * f;
+                sn[c] = io.klast ? yn[c] : yn[c] + io.kamb * f;
+                if (io.klast) wsum += werr_term(bo[c], yn[c], er[c], io.katol, io.krtol);
+              }
+              store_d<VW>(io.kyd, gi, yn);
+              store_d<VW>(io.kerrd, gi, er);
+              store_d<VW>(io.yout, gi, sn);
+              if (io.kfirst) store_d<VW>(io.kbakd, gi, yo);
+            }
+          }
+        }
+      }
+    };
+    if (nel == kQuadEl)
+      update(std::true_type{});
+    else
+      update(std::false_type{});
+    wave_sync();  // su takes the next group's state
+  }
+  if constexpr (EPI == 3 || EPI == 4) {
+    if (io.klast) {
+      // fixed butterfly order: the same sum for the same grid
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) wsum += __shfl_xor(wsum, o, 64);
+      if ((threadIdx.x & 63) == 0) io.kpart[wslot] = wsum;
+    }
+  }
+}
+
+// Compute units of the current device and the blocks of `kernel` (nt threads)
+// resident on one, looked up once per (kernel, device).
+struct Residency {
+  int64_t cus, per_cu;
+};
+inline Residency quad_resident(const void *kernel, int nt) {
+  int dev = 0;
+  RF_HIP(hipGetDevice(&dev));
+  static std::mutex mu;
+  static std::map<std::tuple<const void *, int>, Residency> cache;
+  const auto key = std::make_tuple(kernel, dev);
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    const auto it = cache.find(key);
+    if (it != cache.end()) return it->second;
+  }
+  int cus = 0, per_cu = 0;
+  RF_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  RF_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, nt, 0));
+  const Residency r{cus > 0 ? cus : 1, per_cu > 0 ? per_cu : 1};
+  std::lock_guard<std::mutex> lock(mu);
+  cache.emplace(key, r);
+  return r;
+}
+
+// Blocks and waves per block: the persistent grid, at most the resident
+// blocks. A mesh with fewer groups than a block per compute unit would hold
+// gives fewer waves of each block a group instead of launching fewer blocks,
+// so that its waves do not share a unit while others idle.
+struct QuadGrid {
+  int64_t blocks;
+  int waves;
+};
+template <int NP, bool CIN, int EPI>
+QuadGrid quad_grid(int64_t n_elem) {
+  constexpr int NWB = QuadTab<NP>::NWB;
+  const int64_t groups = (n_elem + kQuadEl - 1) / kQuadEl;
+  const Residency r = quad_resident(reinterpret_cast<const void *>(&k_quad<NP, CIN, EPI>), NWB * 64);
+  const int64_t nw = std::min<int64_t>(NWB, std::max<int64_t>(1, (groups + r.cus - 1) / r.cus));
+  return {std::min((groups + nw - 1) / nw, r.cus * r.per_cu), (int)nw};
+}
+template <int NP, bool CIN, int EPI>
+void quad_launch(const StageArgs &a, hipStream_t s) {
+  const QuadGrid g = quad_grid<NP, CIN, EPI>(a.n_elem);
+  if (g.blocks > 0) hipLaunchKernelGGL((k_quad<NP, CIN, EPI>), dim3((unsigned)g.blocks), dim3(QuadTab<NP>::NWB * 64), 0,
+                       s, a, g.waves);
+}
+template <int NP>
+int64_t quad_slots(bool r64, int64_t n_elem) {
+  const QuadGrid g = r64 ? quad_grid<NP, false, 4>(n_elem) : quad_grid<NP, true, 3>(n_elem);
+  return g.blocks * g.waves;
+}
+template <bool CIN, int EPI>
+void quad_orders(int np, const StageArgs &a, hipStream_t s) {
+  switch (np) {
+    case 4: quad_launch<4, CIN, EPI>(a, s); break;
+    case 10: quad_launch<10, CIN, EPI>(a, s); break;
+    case 20: quad_launch<20, CIN, EPI>(a, s); break;
+    case 35: quad_launch<35, CIN, EPI>(a, s); break;
+    default: throw Error{RFHIP_EUNSUPPORTED, "order not compiled (Np must be 4, 10, 20 or 35)"};
+  }
+  RF_HIP(hipGetLastError());
+}
+
+template <int NP>
+void quad_pack_np(const double *const D[3], const double *lift, std::vector<double> &out) {
+  using T = QuadTab<NP>;
+  using Z = QuadSize<NP>;
+  constexpr int NFP = ElemTab<NP>::NFP, NFR = (Z::NF + 1) / 2;
+  out.assign((size_t)NFR * 32, 0.0);
+  // fragment t, row (contraction) kk, output i: pairs of fragments interleaved
+  auto put = [&](int t, int kk, int i, double v) { out[(size_t)(t / 2) * 32 + (size_t)(4 * kk + i) * 2 + t % 2] = v; };
+  int t = 0;
+  for (int a = 0; a < T::NG; ++a)
+    for (int b = 0; b < T::NG; ++b)
+      for (int k = 0; k < 3; ++k) {
+        if (!quad_nz<NP>(k, a, b)) continue;
+        for (int kk = 0; kk < 4; ++kk)
+          for (int i = 0; i < 4; ++i) {
+            const int r = T::NODE[a][i], c = T::NODE[b][kk];
+            if (r < NP && c < NP) put(t, kk, i, D[k][r * NP + c]);
+          }
+        ++t;
+      }
+  for (int s = 0; s < NFP; ++s)
+    for (int a = 0; a < T::NG; ++a, ++t)
+      for (int kk = 0; kk < 4; ++kk)
+        for (int i = 0; i < 4; ++i) {
+          const int r = T::NODE[a][i];
+          if (r < NP) put(t, kk, i, lift[(size_t)r * 4 * NFP + kk * NFP + s]);
+        }
+}
+}  // namespace
+
+void quad_pack(int np, const double *const D[3], const double *lift, std::vector<double> &out) {
+  switch (np) {
+    case 4: quad_pack_np<4>(D, lift, out); break;
+    case 10: quad_pack_np<10>(D, lift, out); break;
+    case 20: quad_pack_np<20>(D, lift, out); break;
+    case 35: quad_pack_np<35>(D, lift, out); break;
+    default: out.clear();
+  }
+}
+
+void launch_quad(int np, int epi, const StageArgs &a, hipStream_t s) {
+  switch (epi) {
+    case 0: quad_orders<false, 0>(np, a, s); break;
+    case 1: quad_orders<false, 1>(np, a, s); break;
+    case 2: quad_orders<true, 2>(np, a, s); break;
+    case 3: quad_orders<true, 3>(np, a, s); break;
+    default: quad_orders<false, 4>(np, a, s); break;
+  }
+}
+
+int64_t quad_kcl_slots(int np, bool r64, int64_t n_elem) {
+  switch (np) {
+    case 4: return quad_slots<4>(r64, n_elem);
+    case 10: return quad_slots<10>(r64, n_elem);
+    case 20: return quad_slots<20>(r64, n_elem);
+    case 35: return quad_slots<35>(r64, n_elem);
+    default: throw Error{RFHIP_EUNSUPPORTED, "the fused stage kernels run orders 1 to 4"};
+  }
+}
+
+}  // namespace rfhip
