@@ -6,7 +6,9 @@ from the library's own host builder (rfhost_refelem):
   DM[k][i]   bit j set where D_k[i][j] is not zero (k = r, s, t). The host
              builder's D_k carries round-off residues of at most 2e-13 where
              the exact entry is zero (the smallest true entry is 1/3), so the
-             pattern is |D_k[i][j]| > 1e-9 max |D_k|.
+             pattern is |D_k[i][j]| > 1e-9 max |D_k|;
+  XM[k][i]   bit j set where D_k[i][j] is not 0.0 (residues included): the
+             entries that a kernel keeps to add the terms a dense product adds.
 
 The kernel skips the entries outside DM and indexes its per-lane register
 arrays with FN, so both must be known when it is compiled; at operator
@@ -40,6 +42,14 @@ def tables(p: int):
     return r.n_nodes, r.n_face_nodes, r.face_nodes.astype(int).tolist(), masks
 
 
+def exact_masks(p: int):
+    from rapidfem_amd.maxwell import ReferenceElement
+
+    r = ReferenceElement.new(p)
+    return [[sum(1 << j for j in range(d.shape[1]) if d[i, j] != 0.0) for i in range(d.shape[0])]
+            for d in (r.diff_r, r.diff_s, r.diff_t)]
+
+
 def render() -> str:
     out = [
         "// Generated by gen_elem_tables.py from the host builder's reference",
@@ -64,6 +74,10 @@ def render() -> str:
         out.append(f"  static constexpr int FN[4][{nfp}] = {{{rows}}};")
         out.append(f"  static constexpr uint64_t DM[3][{np_}] = {{")
         for mk in masks:
+            out.append("      {" + ", ".join(f"0x{m:x}ull" for m in mk) + "},")
+        out.append("  };")
+        out.append(f"  static constexpr uint64_t XM[3][{np_}] = {{")
+        for mk in exact_masks(p):
             out.append("      {" + ", ".join(f"0x{m:x}ull" for m in mk) + "},")
         out.append("  };")
         out.append("};")

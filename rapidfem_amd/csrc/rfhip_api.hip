@@ -165,21 +165,25 @@ void build_plain(rfhip_op *op, const rfhip_op_desc &d) {
   dv.port = op->port.as<int>();
   dv.perm = op->perm.as<int>();
 }
-// Stage-kernel variant an operator starts with. With FP64 registers k_quad
-// (variant 9) where its table exists: on MI355X it is the fastest at every
-// order from 48 tets to the largest meshes swept (us per stage, fastest other
-// variant against k_quad: 1,296 tets 5.6 / 3.9, 7.6 / 5.4, 9.4 / 8.4,
-// 15.4 / 15.1 at N = 1..4; 1.3M / 768k / 324k / 384k tets 288 / 271,
-// 484 / 350, 416 / 290, 1232 / 687). With compressed registers, whose
-// rounding of p to f32 turns any other order of the sums into differences
-// of the size of that rounding within a few dozen stages, the variants they
-// have always started with (the fastest of the rest per order: pulse boxes of
-// 1.3M / 393k / 324k / 96k tets at N = 1..4), also for operators without the
-// table. autotune re-picks on the operator's own mesh.
+// Stage-kernel variant an operator starts with: k_quad (variant 9) where its
+// tables exist, the fastest on MI355X at every order and both register layouts
+// from 48 tets to the largest meshes swept. us per stage, fastest other variant
+// against k_quad, N = 1..4: FP64 registers, 1,296 tets 5.6 / 3.9, 7.6 / 5.4,
+// 9.4 / 8.4, 15.4 / 15.1; 1.3M / 768k / 324k / 384k tets 288 / 262, 484 / 350,
+// 416 / 290, 1232 / 690; compressed registers, the same large meshes 235 / 221,
+// 410 / 306, 376 / 262, 1170 / 735, with the same bits as the variants named
+// below (their rounding of p to f32 turns any other order of the sums into
+// differences of its own size within a few dozen stages). Compressed registers
+// on small meshes at N = 3, 4, where a stage is one group's chain of operations
+// and that order makes it longer, stay with those variants (1,296 tets: 9.6 /
+// 9.9 and 16.6 / 19.2 us; 3,072: 10.2 / 10.2 and 20.5 / 19.0). Operators without
+// the tables (no permuted node tables, or a state of 2^32 bytes and more) start
+// with the fastest of the rest. autotune re-picks on the operator's own mesh.
 int default_variant(int order, int form, const StageArgs &a) {
   if (form_vmf(form)) return 1;
   const bool c = form == RFHIP_FORM_FUSED_F64C;
-  if (!c && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
+  const bool small = c && order >= 3 && a.n_elem < 2560;
+  if (!small && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
   switch (order) {
     case 1: return c ? 7 : 5;
     case 2: return c ? 7 : 6;
@@ -383,11 +387,14 @@ void build_fused(rfhip_op *op, const rfhip_op_desc &d) {
   if (has_clane) upload(op->clane, clane.data(), clane.size(), s);
   // k_quad (variant 9) on the same element: its fragments and packed node
   // rows. It addresses vectors by 32-bit byte offsets.
-  std::vector<double> quad;
+  std::vector<double> quad, quad_seq;
   std::vector<uint8_t> quad_nodes;
+  bool has_quad_seq = false;
   const bool has_quad = has_clane && 48 * (uint64_t)np * (uint64_t)K < ((uint64_t)1 << 32);
   if (has_quad) {
-    quad_pack(np, D, d.lift, quad);
+    quad_pack(np, D, d.lift, false, quad);
+    has_quad_seq = form_compressed(op->form) && quad_pack(np, D, d.lift, true, quad_seq);
+    if (has_quad_seq) upload(op->quad_seq, quad_seq.data(), quad_seq.size(), s);
     quad_nodes.assign(100 * 16, 0);
     for (int r = 0; r < 100; ++r)
       for (int m = 0; m < nfp; ++m)
@@ -434,6 +441,7 @@ void build_fused(rfhip_op *op, const rfhip_op_desc &d) {
   a.nbase = nbase.empty() ? nullptr : op->nbase.as<int>();
   a.clane = has_clane ? op->clane.as<double>() : nullptr;
   a.quad = has_quad ? op->quad.as<double>() : nullptr;
+  a.quad_seq = has_quad_seq ? op->quad_seq.as<double>() : nullptr;
   a.quad_nodes = has_quad ? op->quad_nodes.p : nullptr;
   a.variant = default_variant(op->order, op->form, a);
 }

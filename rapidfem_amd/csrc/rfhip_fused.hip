@@ -2535,7 +2535,7 @@ bool variant_available(int order, int form, int variant, const StageArgs &a) {
   const int np = (order + 1) * (order + 2) * (order + 3) / 6;
   if (form_vmf(form)) return variant >= 0 && variant < kStageVariantsBf16 && a.nbase != nullptr && order >= 2 && order <= 4;
   if (variant < 0 || variant >= kStageVariants) return false;
-  if (variant == kQuadVariant) return a.quad != nullptr;
+  if (variant == kQuadVariant) return a.quad != nullptr && (!form_compressed(form) || a.quad_seq != nullptr);
   if (variant == 8) return a.clane != nullptr;
   if (variant == 3) return a.nbase != nullptr && np <= 20;
   if (variant >= 4) return a.nbase != nullptr;

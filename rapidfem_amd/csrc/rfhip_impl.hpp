@@ -156,6 +156,7 @@ struct StageArgs {
   const int *nbase;       // [e*4Nfp + fm]: AoS index of the neighbour trace, or the (negative) face code
   const double *clane;    // nonzeros of D_k then LIFT, in k_clane's order (clane_pack), or null
   const double *quad;     // A fragments of D_k's nonzero 4x4 blocks then LIFT, in k_quad's order (quad_pack), or null
+  const double *quad_seq; // the same of the compressed-input kernels, or null
   const void *quad_nodes; // 100 rows of 16 node numbers (bytes): (f*4 + nlf)*6 + orientation, then 96 + f the own face
   const void *yin;        // double, or float hi (compressed)
   const void *yin_lo;     // bf16 lo (compressed) or null
@@ -201,7 +202,7 @@ struct rfhip_op {
   // device operator data
   rfhip::DevBuf dr, ds, dt, lift, face_nodes, jinv, inv_eps, inv_mu, sig_eps, sig_mu, normal, fscale, nbr,
       nbr_lf, port, perm;
-  rfhip::DevBuf dT, liftc, lfrag, afrag7, afragb, clane, quad, quad_nodes, jinv64, fcode, mat, mat_tab, nbr_node, nbase;
+  rfhip::DevBuf dT, liftc, lfrag, afrag7, afragb, clane, quad, quad_seq, quad_nodes, jinv64, fcode, mat, mat_tab, nbr_node, nbase;
   int64_t n_vec = 0;  // length of device vectors (n_dof)
   // Debye dispersive block: slot -> element and (a, g, 1/eps_inf); the P
   // block follows the 6 Np K values of [E,H] in every state vector
@@ -284,13 +285,13 @@ void launch_stage(int order, int form, int epi, const StageArgs &a, hipStream_t 
 // the base variant for them otherwise).
 bool variant_available(int order, int form, int variant, const StageArgs &a);
 // One KCL stage with the register update in the stage kernel's epilogue
-// (k_fused11): with compressed registers (EPI 3) the apply of a.yin /
+// (k_quad, k_fused11): with compressed registers (EPI 3) the apply of a.yin /
 // a.yin_lo, the register update and the next stage's input into a.yout /
 // a.yout_lo; with FP64 registers (r64, EPI 4) the same on a.kyd, a.kerrd,
 // a.kbakd and FP64 stage inputs. Needs the neighbour-trace table and a form
-// without the matrix-core volume; runs variant 6 when a.variant is 6 and
-// variant 7 otherwise. kcl_stage_slots: the number of partial sums the last
-// stage leaves in a.kpart.
+// without the matrix-core volume; runs k_quad when a.variant is 9, variant 6
+// when it is 6 and variant 7 otherwise. kcl_stage_slots: the number of partial
+// sums the last stage leaves in a.kpart.
 bool kcl_stage_fusable(int form, const StageArgs &a);
 int64_t kcl_stage_slots(int order, const StageArgs &a, bool r64);
 void launch_kcl_stage(int order, const StageArgs &a, bool r64, hipStream_t s);
@@ -300,11 +301,12 @@ void launch_kcl_stage(int order, const StageArgs &a, bool r64, hipStream_t s);
 // the zeros of its D_k differ from the compiled equispaced tables.
 bool clane_pack(int np, const int *face_nodes, const double *const D[3], const double *lift, std::vector<double> &out);
 // k_quad (stage-kernel variant 9, rfhip_quad.hip): its fragment table from
-// D_k and LIFT of the compiled equispaced element (clane_pack holds), the
-// launch (epi 0 apply, 1 / 2 LSERK4 stage with FP64 / compressed registers,
+// D_k and LIFT of the compiled equispaced element (clane_pack holds; seq: of
+// the compressed-input kernels, which sum in node order, false where D_k has
+// entries outside the compiled pattern), the launch (epi 0 apply, 1 / 2 LSERK4 stage with FP64 / compressed registers,
 // 3 / 4 KCL stage with compressed / FP64 registers) and the number of partial
 // sums its last KCL stage leaves in a.kpart.
-void quad_pack(int np, const double *const D[3], const double *lift, std::vector<double> &out);
+bool quad_pack(int np, const double *const D[3], const double *lift, bool seq, std::vector<double> &out);
 void launch_quad(int np, int epi, const StageArgs &a, hipStream_t s);
 int64_t quad_kcl_slots(int np, bool r64, int64_t n_elem);
 // Debye block after an applied derivative (dy = A y; f32: plain FP32 form),

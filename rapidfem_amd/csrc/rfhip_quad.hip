@@ -30,12 +30,17 @@
 // one LDS read per 4 x 4 x 16 products instead of one per lane and node) and
 // idle lanes (29 of 64 with one lane per node at N = 4).
 //
+// Compressed registers (CIN) take their sums in node order, by QuadRows: more
+// blocks, the face fluxes formed per node as the one-lane-per-node kernels form
+// them and moved between the lanes (transpose_rows), for the same bits.
+//
 // What bounds it (LSERK4 stage, FP64 registers, 324,000 tets at N = 3, 290 us
 // against 416 for the variant before it): the memory side. Leaving out all
 // products changes nothing, streaming the state and p alone takes 245 us (5.3
 // TB/s), the neighbour traces, 10 M line requests to L2, the rest. At N = 4
-// (384,000 tets, 687 us against 1232) products and vector instructions fill
-// about 70 % of the issue cycles.
+// (384,000 tets, 690 us against 1232) products and vector instructions fill
+// about 70 % of the issue cycles. Compressed registers: 262 us against 376 and
+// 735 against 1170, bound the same way.
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -88,50 +93,86 @@ struct QuadTab<35> {
                                       {24, 12, 13, 14}, {4, 17, 3, 2},   {25, 18, 26, 27}, {32, 35, 31, 34}};
 };
 
-// Whether block (a, b) of D_k has a nonzero.
+// The rows and columns of the products. SEQ: every sum takes its terms in
+// node (and face node) order, as the one-lane-per-node kernels do, entries of
+// D_k that are round-off residues included, so that with v_mfma_f64_4x4x4_4b's
+// chain of FMAs in row order 0..3 the results are theirs bit for bit: the
+// columns are dealt out in order, only the rows into the groups that leave the
+// fewest blocks with entries that are not 0.0 (21 of 27, 66 of 75, 218 of 243).
 template <int NP>
+struct QuadRows;
+template <>
+struct QuadRows<4> {
+  static constexpr int NODE[1][4] = {{0, 1, 2, 3}};
+};
+template <>
+struct QuadRows<10> {
+  static constexpr int NODE[3][4] = {{10, 2, 1, 0}, {5, 10, 3, 4}, {6, 9, 7, 8}};
+};
+template <>
+struct QuadRows<20> {
+  static constexpr int NODE[5][4] = {{16, 19, 10, 17}, {18, 13, 14, 7}, {8, 9, 5, 4}, {3, 0, 2, 1}, {6, 11, 12, 15}};
+};
+template <>
+struct QuadRows<35> {
+  static constexpr int NODE[9][4] = {{4, 1, 2, 3},     {19, 20, 22, 33}, {5, 14, 12, 9}, {27, 26, 17, 16}, {6, 13, 11, 10},
+                                     {32, 25, 18, 15}, {31, 0, 34, 35},  {23, 28, 21, 8}, {30, 7, 24, 29}};
+};
+template <int NP, bool SEQ>
+constexpr int quad_row(int a, int i) {
+  return SEQ ? QuadRows<NP>::NODE[a][i] : QuadTab<NP>::NODE[a][i];
+}
+template <int NP, bool SEQ>
+constexpr int quad_col(int b, int j) {
+  return SEQ ? (4 * b + j < NP ? 4 * b + j : NP) : QuadTab<NP>::NODE[b][j];
+}
+
+// Whether block (a, b) of D_k has a nonzero.
+template <int NP, bool SEQ>
 constexpr bool quad_nz(int k, int a, int b) {
   for (int i = 0; i < 4; ++i)
     for (int j = 0; j < 4; ++j) {
-      const int r = QuadTab<NP>::NODE[a][i], c = QuadTab<NP>::NODE[b][j];
-      if (r < NP && c < NP && ((ElemTab<NP>::DM[k][r] >> c) & 1ull)) return true;
+      const int r = quad_row<NP, SEQ>(a, i), c = quad_col<NP, SEQ>(b, j);
+      if (r < NP && c < NP && (((SEQ ? ElemTab<NP>::XM : ElemTab<NP>::DM)[k][r] >> c) & 1ull)) return true;
     }
   return false;
 }
 // Blocks before (a, b, k) in the order the kernel reads them (k fastest);
-// quad_at<NP>(NG, 0, 0) counts them all and LIFT's fragments start there.
-template <int NP>
+// quad_at(NG, 0, 0) counts them all and LIFT's fragments start there.
+template <int NP, bool SEQ>
 constexpr int quad_at(int a_end, int b_end, int k_end) {
   int s = 0;
   for (int a = 0; a < QuadTab<NP>::NG; ++a)
     for (int b = 0; b < QuadTab<NP>::NG; ++b)
       for (int k = 0; k < 3; ++k) {
         if (a > a_end || (a == a_end && (b > b_end || (b == b_end && k >= k_end)))) return s;
-        s += quad_nz<NP>(k, a, b) ? 1 : 0;
+        s += quad_nz<NP, SEQ>(k, a, b) ? 1 : 0;
       }
   return s;
 }
 // Steps of the volume: the blocks (a, b), a-major, where any D_k has a nonzero.
-template <int NP>
+template <int NP, bool SEQ>
 constexpr int quad_steps() {
   int n = 0;
   for (int ab = 0; ab < QuadTab<NP>::NG * QuadTab<NP>::NG; ++ab)
-    n += quad_nz<NP>(0, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG) || quad_nz<NP>(1, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG) ||
-         quad_nz<NP>(2, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG);
+    n += quad_nz<NP, SEQ>(0, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG) || quad_nz<NP, SEQ>(1, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG) ||
+         quad_nz<NP, SEQ>(2, ab / QuadTab<NP>::NG, ab % QuadTab<NP>::NG);
   return n;
 }
-template <int NP>
+template <int NP, bool SEQ>
 constexpr int quad_step(int st) {
   constexpr int NG = QuadTab<NP>::NG;
   for (int ab = 0; ab < NG * NG; ++ab)
-    if (quad_nz<NP>(0, ab / NG, ab % NG) || quad_nz<NP>(1, ab / NG, ab % NG) || quad_nz<NP>(2, ab / NG, ab % NG))
+    if (quad_nz<NP, SEQ>(0, ab / NG, ab % NG) || quad_nz<NP, SEQ>(1, ab / NG, ab % NG) || quad_nz<NP, SEQ>(2, ab / NG, ab % NG))
       if (st-- == 0) return ab;
   return -1;
 }
-template <int NP>
+template <int NP, bool SEQ>
 struct QuadSize {
-  static constexpr int NV = quad_at<NP>(QuadTab<NP>::NG, 0, 0);
-  static constexpr int NL = ElemTab<NP>::NFP * QuadTab<NP>::NG;
+  static constexpr int NV = quad_at<NP, SEQ>(QuadTab<NP>::NG, 0, 0);
+  // LIFT's column steps: a node of every face, or (SEQ) four nodes of one face
+  static constexpr int NU = (ElemTab<NP>::NFP + 3) / 4;
+  static constexpr int NL = (SEQ ? 4 * NU : ElemTab<NP>::NFP) * QuadTab<NP>::NG;
   static constexpr int NF = NV + NL;  // A fragments of 16 doubles
 };
 
@@ -151,13 +192,40 @@ __device__ __forceinline__ double other_field(double v) {
   return __builtin_bit_cast(double, make_int2(lo, hi));
 }
 
-// Two floats to bf16 (round to nearest even), a in the low half. As an
-// instruction of its own: from (float)double operands the compiler forms an
-// f64 -> bf16 conversion of six vector instructions and a branch per value.
+// The 4x4 transpose of four registers over the four rows of 16 lanes: row q of
+// register f takes row f of register q.
+__device__ __forceinline__ void transpose_rows(double &r0, double &r1, double &r2, double &r3) {
+  uint2 v[4] = {__builtin_bit_cast(uint2, r0), __builtin_bit_cast(uint2, r1), __builtin_bit_cast(uint2, r2),
+                __builtin_bit_cast(uint2, r3)};
+  auto half = [](uint32_t &a, uint32_t &b) {  // rows 2, 3 of a with rows 0, 1 of b
+    const auto t = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = t[0];
+    b = t[1];
+  };
+  auto quarter = [](uint32_t &a, uint32_t &b) {  // rows 1, 3 of a with rows 0, 2 of b
+    const auto t = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = t[0];
+    b = t[1];
+  };
+  half(v[0].x, v[2].x);
+  half(v[1].x, v[3].x);
+  half(v[0].y, v[2].y);
+  half(v[1].y, v[3].y);
+  quarter(v[0].x, v[1].x);
+  quarter(v[2].x, v[3].x);
+  quarter(v[0].y, v[1].y);
+  quarter(v[2].y, v[3].y);
+  r0 = __builtin_bit_cast(double, v[0]);
+  r1 = __builtin_bit_cast(double, v[1]);
+  r2 = __builtin_bit_cast(double, v[2]);
+  r3 = __builtin_bit_cast(double, v[3]);
+}
+
+// Two floats to bf16 (round to nearest even), a in the low half, as in
+// rfhip_fused.hip (from (float)double operands the compiler rounds once).
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
-  uint32_t r;
-  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-  return r;
+  const __bf16 x = (__bf16)a, y = (__bf16)b;
+  return (uint32_t)__builtin_bit_cast(uint16_t, x) | ((uint32_t)__builtin_bit_cast(uint16_t, y) << 16);
 }
 __device__ __forceinline__ double c_f64(float h, uint32_t lo_bits) { return (double)h + (double)__uint_as_float(lo_bits); }
 
@@ -348,9 +416,12 @@ __device__ __forceinline__ int64_t quad_block() {
 // Waves per SIMD the registers are fitted to: the most that leave no spills
 // (N = 2: 300 us at 3 waves, 342 at 2 with compressed registers; 427 at 3 with
 // 13 spilled, 350 at 2, with FP64 ones; N = 3 at 3 waves spills 48 to 100).
+// N = 1 takes 4 although 3 stream a large mesh faster (262 us against 271 for
+// 1.3M tets): up to 32,768 tets every group then runs at once (27,030 tets: 9.8
+// us per stage against 11.4).
 template <int NP, int EPI>
 struct QuadWaves {
-  static constexpr int v = NP == 4 ? 4 : NP == 10 && (EPI == 0 || EPI == 2) ? 3 : 2;
+  static constexpr int v = NP == 4 ? (EPI <= 2 ? 4 : 3) : NP == 10 && (EPI == 0 || EPI == 2) ? 3 : 2;
 };
 
 // EPI as in the other stage kernels: 0 apply, 1 LSERK4 stage with FP64
@@ -360,7 +431,8 @@ struct QuadWaves {
 template <int NP, bool CIN, int EPI>
 __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_waves_per_eu(QuadWaves<NP, EPI>::v))) k_quad(StageArgs io, int nw) {
   using T = QuadTab<NP>;
-  using Z = QuadSize<NP>;
+  constexpr bool SEQ = CIN;
+  using Z = QuadSize<NP, SEQ>;
   constexpr int NG = T::NG, NT = T::NWB * 64, NFP = ElemTab<NP>::NFP;
   constexpr int SE = 6 * NP;             // values per element
   constexpr int SW = kQuadEl * SE;       // values per group
@@ -374,11 +446,15 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
   constexpr int NFR = (Z::NF + 1) / 2;   // fragment pairs
   __shared__ __align__(16) double sA[NFR * 32];
   __shared__ __align__(16) uint4 snode[100];
-  __shared__ int splace[4 * NG];
+  __shared__ int splace[2][4 * NG];  // LDS place in an element of column (0) and row (1) node (g, q)
   __shared__ __align__(16) double su_b[T::NWB][SZ + 8];  // + zeros the padding nodes read, + a place for what they write
-  for (int t = threadIdx.x; t < NFR * 16; t += NT) reinterpret_cast<double2 *>(sA)[t] = reinterpret_cast<const double2 *>(io.quad)[t];
+  for (int t = threadIdx.x; t < NFR * 16; t += NT) reinterpret_cast<double2 *>(sA)[t] = reinterpret_cast<const double2 *>(SEQ ? io.quad_seq : io.quad)[t];
   for (int t = threadIdx.x; t < 100; t += NT) snode[t] = reinterpret_cast<const uint4 *>(io.quad_nodes)[t];
-  if ((int)threadIdx.x < 4 * NG) splace[threadIdx.x] = 6 * T::NODE[threadIdx.x / 4][threadIdx.x % 4];
+  if ((int)threadIdx.x < 4 * NG) {
+    const int g = threadIdx.x >> 2, r = threadIdx.x & 3;
+    splace[1][threadIdx.x] = 6 * quad_row<NP, SEQ>(g, r);
+    splace[0][threadIdx.x] = 6 * quad_col<NP, SEQ>(g, r);
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   double *su = su_b[wave];
@@ -405,12 +481,12 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
   const double2 *fr = reinterpret_cast<const double2 *>(sA) + (4 * q + (lane & 3));
   // LDS index of this lane's three values at node(g, q), from a table where
   // they are used (held for the whole group they would cost NG registers).
-  auto places = [&](int (&un)[NG]) {
+  auto places = [&](int (&un)[NG], int rc) {
     int t = q;
     asm volatile("" : "+v"(t));
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      const int n = splace[4 * g + t];
+      const int n = splace[rc][4 * g + t];
       un[g] = n < SE ? el * SP + n + 3 * fld : SZ;
     }
   };
@@ -541,19 +617,19 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
     double acc[NG][3];
     double ub[2][3];
     int un[NG];
-    places(un);
+    places(un, 0);
     auto operand = [&](auto bc) {
       constexpr int st = bc;  // step: block (a, b) = (quad_step / NG, quad_step % NG)
-      constexpr int ab = quad_step<NP>(st);
+      constexpr int ab = quad_step<NP, SEQ>(st);
 #pragma unroll
       for (int c = 0; c < 3; ++c) ub[st & 1][c] = su[un[ab % NG] + c];
     };
-    constexpr int NST = quad_steps<NP>();
+    constexpr int NST = quad_steps<NP, SEQ>();
     operand(std::integral_constant<int, 0>{});
     double r[3][3];
     unroll<0, NST>([&](auto sc) {
-      constexpr int st = sc, ab = quad_step<NP>(st), a = ab / NG, b = ab % NG;
-      if constexpr (st == 0 || quad_step<NP>(st - 1) / NG != a) {
+      constexpr int st = sc, ab = quad_step<NP, SEQ>(st), a = ab / NG, b = ab % NG;
+      if constexpr (st == 0 || quad_step<NP, SEQ>(st - 1) / NG != a) {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
 #pragma unroll
@@ -562,14 +638,19 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
       if constexpr (st + 1 < NST) operand(std::integral_constant<int, st + 1>{});
       unroll<0, 3>([&](auto kc) {
         constexpr int k = kc;
-        if constexpr (quad_nz<NP>(k, a, b)) {
-          const double f = frag(std::integral_constant<int, quad_at<NP>(a, b, k)>{});
+        if constexpr (quad_nz<NP, SEQ>(k, a, b)) {
+          const double f = frag(std::integral_constant<int, quad_at<NP, SEQ>(a, b, k)>{});
 #pragma unroll
           for (int c = 0; c < 3; ++c) r[k][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(f, ub[st & 1][c], r[k][c], 0, 0, 0);
         }
       });
-      if constexpr (st + 1 == NST || quad_step<NP>(st + 1) / NG != a) {
-        auto pd = [&](int p, int c) { return ji[p] * r[0][c] + ji[3 + p] * r[1][c] + ji[6 + p] * r[2][c]; };
+      if constexpr (st + 1 == NST || quad_step<NP, SEQ>(st + 1) / NG != a) {
+        auto pd = [&](int p, int c) {
+          double t = fma(ji[p], r[0][c], ji[3 + p] * r[1][c]);
+          // k_fused9 at Np = 35 starts E_x's two sums with the other product
+          if (SEQ && NP == 35 && c == 0) t = fld ? t : fma(ji[3 + p], r[1][c], ji[p] * r[0][c]);
+          return fma(ji[6 + p], r[2][c], t);
+        };
         acc[a][0] = other_field(pd(1, 2) - pd(2, 1));
         acc[a][1] = other_field(pd(2, 0) - pd(0, 2));
         acc[a][2] = other_field(pd(0, 1) - pd(1, 0));
@@ -588,6 +669,7 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
       nncode = io.fcode[4 * e2 + q];
       nnmat = io.mat[e2];
     }
+    constexpr bool kLateRegs = T::LATE || EPI == 4;
     Upd<EPI, VW> up[EPI == 0 ? 1 : IT];
     auto read_registers = [&] {
       if constexpr (EPI != 0) {
@@ -599,32 +681,15 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
         }
       }
     };
-    if constexpr (!T::LATE) read_registers();
+    if constexpr (!kLateRegs) read_registers();
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
 
-    // Face geometry: m = -+ 0.5 g = -+ cf n of face q (sign as ji), cf = |m|.
-    double m[3];
-    // m = a row of J^-1 or their sum: weights 0, +-1/2 per lane, without branches
-    const double wr0 = q == 1 ? -0.5 : q == 3 ? 0.5 : 0.0, wr1 = q == 2 ? -0.5 : q == 3 ? 0.5 : 0.0,
-                 wr2 = q == 0 ? -0.5 : q == 3 ? 0.5 : 0.0;
-#pragma unroll
-    for (int x = 0; x < 3; ++x) m[x] = wr0 * ji[x] + wr1 * ji[3 + x] + wr2 * ji[6 + x];
-    const double ss = m[0] * m[0] + m[1] * m[1] + m[2] * m[2], hs = 0.5 * ss;
-    double ic = __builtin_amdgcn_rsq(ss);  // 1 / cf, two Newton steps as in face_geom
-    ic = ic * fma(-hs * ic, ic, 1.5);
-    ic = ic * fma(-hs * ic, ic, 1.5);
-    const double al = code < kCodePec ? 1.0 : io.alpha;
-    const double acf = al * (ss * ic), aic = al * ic;
-
-    // Flux and LIFT, one face node of every face at a time:
-    // F = m (m . j) a / cf - a cf j -+ m x j' (j: this field's jump, j' the
-    // other's), j = own + sx * neighbour. On a boundary face the trace read is
-    // the own one, and since F keeps the tangential part of either jump, the
-    // wall and port rules are this sign: PEC ([E] = 2 E_t, [H] = 2 H_n: j = 2 E
-    // and 0), port ([.] = the own trace). The flux of a node is formed while
-    // the products of the node before it run.
-    const double sx = code >= 0 ? -1.0 : code < kCodePec ? 0.0 : fld ? -1.0 : 1.0;
+    D3 minv, msig;
+    auto read_materials = [&] {
+      minv = ld<D3>(io.mat_tab, 96 * (uint32_t)mat + 24 * fld);
+      msig = ld<D3>(io.mat_tab, 96 * (uint32_t)mat + 48 + 24 * fld);
+    };
     const double *const us = su + el * SP + 3 * fld;
     int qo = 96 + q;
     asm volatile("" : "+v"(qo));  // not a loop constant held in registers
@@ -636,28 +701,105 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
       ow[1] = p[1];
       ow[2] = p[2];
     };
-    D3 minv, msig;
-    {
+    // The jump j = own + sx * neighbour of slot s in this lane's field. On a
+    // boundary face the trace read is the own one, and since the flux keeps
+    // the tangential part of either jump, the wall and port rules are this
+    // sign: PEC j = E (doubled in the flux) and 0, port j = own.
+    auto jump = [&](auto sc, double sx, double (&j)[3]) {
+      constexpr int s = sc;
+      const Trace<CIN> x = tr[s % NTR];
+      if constexpr (CIN) {
+        const uint32_t sh = fld << 4;
+        const uint32_t l0 = __builtin_amdgcn_alignbit(x.l.y, x.l.x, sh), l1 = x.l.y >> sh;
+        j[0] = fma(sx, c_f64(x.h.x, l0 << 16), ow[0]);
+        j[1] = fma(sx, c_f64(x.h.y, l0 & 0xFFFF0000u), ow[1]);
+        j[2] = fma(sx, c_f64(x.h.z, l1 << 16), ow[2]);
+      } else {
+        j[0] = fma(sx, x.d.x, ow[0]);
+        j[1] = fma(sx, x.d.y, ow[1]);
+        j[2] = fma(sx, x.d.z, ow[2]);
+      }
+      if constexpr (ROLL && s + TW < NFP) load_trace(s + TW);
+      if constexpr (s + 1 < NFP) own_trace(s + 1);
+    };
+    // Weights 0, +-1 per lane that make face q's vector of J^-1's rows without
+    // branches; the sums of the other rows' zeros are exact.
+    const double wr0 = q == 1 ? -1.0 : q == 3 ? 1.0 : 0.0, wr1 = q == 2 ? -1.0 : q == 3 ? 1.0 : 0.0,
+                 wr2 = q == 0 ? -1.0 : q == 3 ? 1.0 : 0.0;
+    if constexpr (SEQ) {
+      // The operations and their order are face_geom's and face_flux's. n has
+      // this lane's sign (E: -n), which the products n (n.j) do not see.
+      double g[3];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) g[x] = fma(wr2, ji[6 + x], fma(wr0, ji[x], wr1 * ji[3 + x]));
+      const double gs = fma(g[2], g[2], fma(g[0], g[0], g[1] * g[1])), hs = 0.5 * gs;
+      double iy = __builtin_amdgcn_rsq(gs);
+      iy = iy * fma(-hs * iy, iy, 1.5);
+      iy = iy * fma(-hs * iy, iy, 1.5);
+      const double n0 = g[0] * iy, n1 = g[1] * iy, n2 = g[2] * iy;
+      const bool pec = code == kCodePec;
+      const double cf = (pec ? (fld ? 2.0 : 2.0 * io.alpha) : 1.0) * (hs * iy);
+      const double al = code < 0 ? 1.0 : io.alpha;
+      const double sx = code >= 0 ? -1.0 : pec && fld ? -1.0 : 0.0;
+      double F[4 * Z::NU][3];
+      own_trace(0);
+      unroll<0, 4 * Z::NU>([&](auto sc) {
+        constexpr int s = sc;
+        if constexpr (s < NFP) {
+          double j[3], o[3];
+          jump(sc, sx, j);
+#pragma unroll
+          for (int c = 0; c < 3; ++c) o[c] = other_field(j[c]);
+          const double nj = fma(n2, j[2], fma(n0, j[0], n1 * j[1]));
+          F[s][0] = cf * fma(al, fma(n0, nj, -j[0]), fma(n1, o[2], -(n2 * o[1])));
+          F[s][1] = cf * fma(al, fma(n1, nj, -j[1]), fma(n2, o[0], -(n0 * o[2])));
+          F[s][2] = cf * fma(al, fma(n2, nj, -j[2]), fma(n0, o[1], -(n1 * o[0])));
+        } else {
+          F[s][0] = F[s][1] = F[s][2] = 0.0;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      // Four nodes of four faces: from (node, lane = face) to (face, lane = node).
+#pragma unroll
+      for (int u = 0; u < Z::NU; ++u)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) transpose_rows(F[4 * u][c], F[4 * u + 1][c], F[4 * u + 2][c], F[4 * u + 3][c]);
+      unroll<0, 4>([&](auto fc) {
+        unroll<0, Z::NU>([&](auto uc) {
+          constexpr int f = fc, u = uc;
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (f == 3 && u == 0) read_materials();
+          unroll<0, NG>([&](auto ac) {
+            constexpr int a = ac;
+            const double w = frag(std::integral_constant<int, Z::NV + (f * Z::NU + u) * NG + a>{});
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+              acc[a][c] = __builtin_amdgcn_mfma_f64_4x4x4f64(w, F[4 * u + f][c], acc[a][c], 0, 0, 0);
+          });
+        });
+      });
+    } else {
+      // m = -+ 0.5 g = -+ cf n of face q (sign as ji), cf = |m|.
+      double m[3];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) m[x] = 0.5 * (wr0 * ji[x] + wr1 * ji[3 + x] + wr2 * ji[6 + x]);
+      const double ss = m[0] * m[0] + m[1] * m[1] + m[2] * m[2], hs = 0.5 * ss;
+      double ic = __builtin_amdgcn_rsq(ss);  // 1 / cf, two Newton steps as in face_geom
+      ic = ic * fma(-hs * ic, ic, 1.5);
+      ic = ic * fma(-hs * ic, ic, 1.5);
+      const double al = code < kCodePec ? 1.0 : io.alpha;
+      const double acf = al * (ss * ic), aic = al * ic;
+      // Flux and LIFT, one face node of every face at a time:
+      // F = m (m . j) a / cf - a cf j -+ m x j' (j: this field's jump, j' the
+      // other's; PEC j = 2 E and 0). The flux of a node is formed while the
+      // products of the node before it run.
+      const double sx = code >= 0 ? -1.0 : code < kCodePec ? 0.0 : fld ? -1.0 : 1.0;
       double F[2][3];
       own_trace(0);
       auto flux = [&](auto sc) {
         constexpr int s = sc;
-        double j[3];
-        const Trace<CIN> x = tr[s % NTR];
-        if constexpr (CIN) {
-          const uint32_t sh = fld << 4;
-          const uint32_t l0 = __builtin_amdgcn_alignbit(x.l.y, x.l.x, sh), l1 = x.l.y >> sh;
-          j[0] = fma(sx, c_f64(x.h.x, l0 << 16), ow[0]);
-          j[1] = fma(sx, c_f64(x.h.y, l0 & 0xFFFF0000u), ow[1]);
-          j[2] = fma(sx, c_f64(x.h.z, l1 << 16), ow[2]);
-        } else {
-          j[0] = fma(sx, x.d.x, ow[0]);
-          j[1] = fma(sx, x.d.y, ow[1]);
-          j[2] = fma(sx, x.d.z, ow[2]);
-        }
-        if constexpr (ROLL && s + TW < NFP) load_trace(s + TW);
-        if constexpr (s + 1 < NFP) own_trace(s + 1);
-        double o[3];
+        double j[3], o[3];
+        jump(sc, sx, j);
 #pragma unroll
         for (int c = 0; c < 3; ++c) o[c] = other_field(j[c]);
         const double t = aic * (m[0] * j[0] + m[1] * j[1] + m[2] * j[2]);
@@ -669,10 +811,7 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
       unroll<0, NFP>([&](auto sc) {
         constexpr int s = sc;
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (s == (NFP > 3 ? NFP - 3 : 0)) {
-          minv = ld<D3>(io.mat_tab, 96 * (uint32_t)mat + 24 * fld);
-          msig = ld<D3>(io.mat_tab, 96 * (uint32_t)mat + 48 + 24 * fld);
-        }
+        if constexpr (s == (NFP > 3 ? NFP - 3 : 0)) read_materials();
         if constexpr (s + 1 < NFP) flux(std::integral_constant<int, s + 1>{});
         unroll<0, NG>([&](auto ac) {
           constexpr int a = ac;
@@ -685,17 +824,23 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
 
     // Materials (rhs.rs:1443-1454), then the right-hand side to LDS in place
     // of the state, which the update takes into registers first.
+    auto rhs = [](double mi, double a, double ms, double u) {
+      if constexpr (SEQ)
+        return fma(mi, a, -(ms * u));
+      else
+        return mi * a - ms * u;
+    };
     int up_at[NG];
-    places(up_at);
+    places(up_at, 1);
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
-      acc[g][0] = minv.x * acc[g][0] - msig.x * su[up_at[g]];
-      acc[g][1] = minv.y * acc[g][1] - msig.y * su[up_at[g] + 1];
-      acc[g][2] = minv.z * acc[g][2] - msig.z * su[up_at[g] + 2];
+      acc[g][0] = rhs(minv.x, acc[g][0], msig.x, su[up_at[g]]);
+      acc[g][1] = rhs(minv.y, acc[g][1], msig.y, su[up_at[g] + 1]);
+      acc[g][2] = rhs(minv.z, acc[g][2], msig.z, su[up_at[g] + 2]);
     }
     // the next group's geometry and traces, ahead of this group's stores
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (T::LATE) read_registers();
+    if constexpr (kLateRegs) read_registers();
     code = ncode;
     mat = nmat;
     read_geom(grp1, code);
@@ -718,7 +863,8 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
     wave_sync();
     unroll<0, NG>([&](auto gc) {
       constexpr int g = gc;
-      constexpr bool pad = T::NODE[g][0] >= NP || T::NODE[g][1] >= NP || T::NODE[g][2] >= NP || T::NODE[g][3] >= NP;
+      constexpr bool pad = quad_row<NP, SEQ>(g, 0) >= NP || quad_row<NP, SEQ>(g, 1) >= NP ||
+                           quad_row<NP, SEQ>(g, 2) >= NP || quad_row<NP, SEQ>(g, 3) >= NP;
       const int to = pad && up_at[g] >= SZ ? SZ + 4 : up_at[g];
 #pragma unroll
       for (int c = 0; c < 3; ++c) su[to + c] = acc[g][c];
@@ -726,7 +872,7 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
     wave_sync();
     const int nv = nel * SE;
     auto update = [&](auto full) {
-      constexpr int CH = 4;  // iterations of right-hand sides in registers at a time
+      constexpr int CH = T::LATE ? 2 : 4;  // iterations of right-hand sides in registers at a time
 #pragma unroll
       for (int k0 = 0; k0 < IT; k0 += CH) {
         double kr[CH][VW];
@@ -779,8 +925,12 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
               double yn[VW];
     #pragma unroll
               for (int c = 0; c < VW; ++c) {
-                pn[c] = (float)(io.sa * (double)up[k].p.v[c] + io.dt * kv[c]);
-                yn[c] = yv[k][c] + io.sb * (double)pn[c];
+                // which product is rounded on its own: dt k in E_x (i = 0 mod 6), a p in the rest
+                const double po = up[k].p.v[c];
+                double v = fma(io.dt, kv[c], io.sa * po);
+                if (c % 2 == 0) v = (i + c) % 6 == 0 ? fma(io.sa, po, io.dt * kv[c]) : v;
+                pn[c] = (float)v;
+                yn[c] = fma(io.sb, (double)pn[c], yv[k][c]);
               }
               store_f<VW>(io.p, gi, pn);
               store_c<VW>(io.yout, io.yout_lo, gi, yn);
@@ -909,43 +1059,64 @@ void quad_orders(int np, const StageArgs &a, hipStream_t s) {
   RF_HIP(hipGetLastError());
 }
 
-template <int NP>
+template <int NP, bool SEQ>
 void quad_pack_np(const double *const D[3], const double *lift, std::vector<double> &out) {
-  using T = QuadTab<NP>;
-  using Z = QuadSize<NP>;
-  constexpr int NFP = ElemTab<NP>::NFP, NFR = (Z::NF + 1) / 2;
+  using Z = QuadSize<NP, SEQ>;
+  constexpr int NG = QuadTab<NP>::NG, NFP = ElemTab<NP>::NFP, NFR = (Z::NF + 1) / 2;
   out.assign((size_t)NFR * 32, 0.0);
   // fragment t, row (contraction) kk, output i: pairs of fragments interleaved
   auto put = [&](int t, int kk, int i, double v) { out[(size_t)(t / 2) * 32 + (size_t)(4 * kk + i) * 2 + t % 2] = v; };
   int t = 0;
-  for (int a = 0; a < T::NG; ++a)
-    for (int b = 0; b < T::NG; ++b)
+  for (int a = 0; a < NG; ++a)
+    for (int b = 0; b < NG; ++b)
       for (int k = 0; k < 3; ++k) {
-        if (!quad_nz<NP>(k, a, b)) continue;
+        if (!quad_nz<NP, SEQ>(k, a, b)) continue;
         for (int kk = 0; kk < 4; ++kk)
           for (int i = 0; i < 4; ++i) {
-            const int r = T::NODE[a][i], c = T::NODE[b][kk];
+            const int r = quad_row<NP, SEQ>(a, i), c = quad_col<NP, SEQ>(b, kk);
             if (r < NP && c < NP) put(t, kk, i, D[k][r * NP + c]);
           }
         ++t;
       }
-  for (int s = 0; s < NFP; ++s)
-    for (int a = 0; a < T::NG; ++a, ++t)
-      for (int kk = 0; kk < 4; ++kk)
+  // LIFT: the columns of step s are node s of every face, or (SEQ) four nodes
+  // of one face in turn, the last step of a face filled up with zeros
+  for (int s = 0; s < (SEQ ? 4 * Z::NU : NFP); ++s)
+    for (int a = 0; a < NG; ++a, ++t)
+      for (int kk = 0; kk < 4; ++kk) {
+        const int f = SEQ ? s / Z::NU : kk, m = SEQ ? 4 * (s % Z::NU) + kk : s;
         for (int i = 0; i < 4; ++i) {
-          const int r = T::NODE[a][i];
-          if (r < NP) put(t, kk, i, lift[(size_t)r * 4 * NFP + kk * NFP + s]);
+          const int r = quad_row<NP, SEQ>(a, i);
+          if (r < NP && m < NFP) put(t, kk, i, lift[(size_t)r * 4 * NFP + f * NFP + m]);
         }
+      }
+}
+// Whether every entry of D_k that is not 0.0 is one the SEQ kernels keep.
+template <int NP>
+bool quad_exact_np(const double *const D[3]) {
+  for (int k = 0; k < 3; ++k)
+    for (int i = 0; i < NP; ++i)
+      for (int j = 0; j < NP; ++j)
+        if (D[k][i * NP + j] != 0.0 && !((ElemTab<NP>::XM[k][i] >> j) & 1ull)) return false;
+  return true;
+}
+template <int NP>
+bool quad_pack_both(const double *const D[3], const double *lift, bool seq, std::vector<double> &out) {
+  if (seq && !quad_exact_np<NP>(D)) return false;
+  if (seq)
+    quad_pack_np<NP, true>(D, lift, out);
+  else
+    quad_pack_np<NP, false>(D, lift, out);
+  return true;
 }
 }  // namespace
 
-void quad_pack(int np, const double *const D[3], const double *lift, std::vector<double> &out) {
+bool quad_pack(int np, const double *const D[3], const double *lift, bool seq, std::vector<double> &out) {
   switch (np) {
-    case 4: quad_pack_np<4>(D, lift, out); break;
-    case 10: quad_pack_np<10>(D, lift, out); break;
-    case 20: quad_pack_np<20>(D, lift, out); break;
-    case 35: quad_pack_np<35>(D, lift, out); break;
-    default: out.clear();
+    case 4: return quad_pack_both<4>(D, lift, seq, out);
+    case 10: return quad_pack_both<10>(D, lift, seq, out);
+    case 20: return quad_pack_both<20>(D, lift, seq, out);
+    case 35: return quad_pack_both<35>(D, lift, seq, out);
+    default: return false;
   }
 }
 

@@ -88,3 +88,37 @@ def test_kcl_on_partial_groups_matches_oracle(ctx, oracle, order, k):
         if mode == "f64":
             assert (st.accepted, st.rejected) == (acc, rej)
         assert err < (1e-11 if mode == "f64" else 1e-6)
+
+
+@pytest.mark.parametrize("alpha", [1.0, 0.7, 0.0])
+@pytest.mark.parametrize("order, other", [(1, 7), (2, 7), (3, 7), (4, 4)])
+def test_compressed_registers_keep_every_bit(ctx, oracle, order, other, alpha):
+    """With compressed registers k_quad takes every sum in the order of the
+    one-lane-per-node kernels: 40 steps leave the same bits. In the second run
+    a held source -A y leaves the rounding of the first stage's right-hand side
+    as the whole of p, so its last FP64 bit shows."""
+    from rapidfem_amd import Drive, GpuOperator
+
+    k = 129
+    xyz, tets = oracle.box_mesh(3, 3, 3, 1.0, 1.0, 1.0, 0.1, 7, True)
+    rng = np.random.default_rng(order)
+    port = np.where(rng.random(4 * k) < 0.3, 0, -1).astype(np.int32)
+    oop = oracle.Operator(xyz, tets.reshape(-1, 4)[:k], order, alpha, eps=rng.uniform(1, 4, (k, 3)),
+                          sigma=rng.uniform(0, 1, k), face_port=port)
+    y = rng.normal(size=oop.n_dof)
+    d, arrs, re_, ex = oracle_desc(oop)
+    g = GpuOperator.from_desc(ctx, d, "fused_f64c", mass=re_["mass"], det=ex["det"])
+    got = []
+    for v in (other, QUAD):
+        g.set_variant(v)
+        g.poison_lds()
+        got.append(g.transient(ctx, y, 0.001, 40, 1, Drive.point(3), np.linspace(0, 1, 40), record=False,
+                               precision="f64"))
+    assert np.array_equal(got[0], got[1])
+    y = np.ldexp(y.astype(np.float32).astype(np.float64), -60)
+    src = -g.apply_f64(y)
+    got = []
+    for v in (other, QUAD):
+        g.set_variant(v)
+        got.append(g.transient(ctx, y, 1e8, 1, 1, Drive.vector(src), np.ones(1), record=False, precision="f64"))
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0], got[1])
