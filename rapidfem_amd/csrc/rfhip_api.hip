@@ -176,14 +176,17 @@ void build_plain(rfhip_op *op, const rfhip_op_desc &d) {
 // differences of its own size within a few dozen stages). Compressed registers
 // on small meshes at N = 3, 4, where a stage is one group's chain of operations
 // and that order makes it longer, stay with those variants (1,296 tets: 9.6 /
-// 9.9 and 16.6 / 19.2 us; 3,072: 10.2 / 10.2 and 20.5 / 19.0). Operators without
+// 9.9 and 16.6 / 19.2 us; 3,072: 10.2 / 10.2 and 20.5 / 19.0), and so do they at
+// N = 1 between the size where every group runs at once and the one where the
+// state no longer fits the 256 MB cache (17,640 tets 9.0 / 7.6, 27,648 8.2 / 8.8,
+// 196,608 33 / 36, 384,000 61 / 67, 750,000 139 / 125). Operators without
 // the tables (no permuted node tables, or a state of 2^32 bytes and more) start
 // with the fastest of the rest. autotune re-picks on the operator's own mesh.
 int default_variant(int order, int form, const StageArgs &a) {
   if (form_vmf(form)) return 1;
   const bool c = form == RFHIP_FORM_FUSED_F64C;
-  const bool small = c && order >= 3 && a.n_elem < 2560;
-  if (!small && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
+  const bool keep = c && (order >= 3 ? a.n_elem < 2560 : order == 1 && a.n_elem > 24576 && a.n_elem < 700000);
+  if (!keep && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
   switch (order) {
     case 1: return c ? 7 : 5;
     case 2: return c ? 7 : 6;
