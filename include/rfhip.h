@@ -258,7 +258,7 @@ int rfhip_op_transient_kcl_f64(rfhip_op *op, const double *y0, double dt,
 int rfhip_op_set_kcl_registers(rfhip_op *op, int32_t mode);
 
 /* GpuOperator::expmv (gpu/operator.rs:1175-1197): out = exp(t*A)*v, FP64
- * Arnoldi (CGS2) with the Hessenberg exponential, following
+ * Arnoldi (DCGS2) with the Hessenberg exponential, following
  * propagator.rs:186-326: max_dim caps the dimension, tol > 0 enables the
  * a-posteriori stop (0 = fixed dimension). The basis is held whole in HBM,
  * so no KRYLOV_CHUNK sub-stepping. dim_used may be NULL. */

@@ -834,10 +834,11 @@ void kcl_impl(rfhip_op *op, void *ys, double dt, int64_t steps, int kind, int64_
 
 // ---- Krylov (propagator.rs:186-373) ---------------------------------------
 
-// Arnoldi with CGS2 on the device, Hessenberg on the host. aug: the ETD
-// augmentation [[A, b], [0, 0]] with the scalar component carried here and
-// b = op->src (a layout vector).
-int krylov_impl(rfhip_op *op, const double *v_host, double t, int max_dim, double tol, bool aug, double *out) {
+// Arnoldi with CGS2 on the device, Hessenberg on the host: the path of inputs
+// with non-finite products, whose infinities and NaN it carries to the
+// result. aug: the ETD augmentation [[A, b], [0, 0]] with the scalar
+// component carried here and b = op->src (a layout vector).
+int krylov_cgs2(rfhip_op *op, const double *v_host, double t, int max_dim, double tol, bool aug, double *out) {
   const int64_t n = nvec(op);
   RF_REQUIRE(max_dim >= 1 && max_dim <= kMaxKrylov, "Krylov dimension must be in [1, 64]");
   hipStream_t s = op->stream;
@@ -895,15 +896,15 @@ int krylov_impl(rfhip_op *op, const double *v_host, double t, int max_dim, doubl
     double ws = 0.0;  // augmented scalar of w (zero row of the augmented matrix)
     const int cols = j + 1;
     double norm2 = 0.0;
-    // Classical Gram-Schmidt, two passes. The first pass's update and the
-    // second pass's projections share one sweep over the basis.
+    // Classical Gram-Schmidt, two passes.
     launch_multi_dot(basis, n, cols, w, part, nblk, proj, s);
     if (!aug) {
       // The host only accumulates H here: both passes' projections and the
       // norm come back asynchronously, one wait per step.
       double *hp = op->kb_host.as<double>();
       RF_HIP(hipMemcpyAsync(hp, proj, 8 * cols, hipMemcpyDeviceToHost, s));
-      launch_axpy_dot(w, basis, n, cols, proj, part, nblk, proj, s);
+      launch_axpy_basis_norm(w, basis, n, cols, proj, part, nblk, norm_dev, s);
+      launch_multi_dot(basis, n, cols, w, part, nblk, proj, s);
       RF_HIP(hipMemcpyAsync(hp + kMaxKrylov, proj, 8 * cols, hipMemcpyDeviceToHost, s));
       launch_axpy_basis_norm(w, basis, n, cols, proj, part, nblk, norm_dev, s);
       RF_HIP(hipMemcpyAsync(hp + 2 * kMaxKrylov, norm_dev, 8, hipMemcpyDeviceToHost, s));
@@ -919,7 +920,8 @@ int krylov_impl(rfhip_op *op, const double *v_host, double t, int max_dim, doubl
       // second pass waits for the host.
       double *hp = op->kb_host.as<double>();
       RF_HIP(hipMemcpyAsync(hp, proj, 8 * cols, hipMemcpyDeviceToHost, s));
-      launch_axpy_dot(w, basis, n, cols, proj, part, nblk, proj, s);
+      launch_axpy_basis_norm(w, basis, n, cols, proj, part, nblk, norm_dev, s);
+      launch_multi_dot(basis, n, cols, w, part, nblk, proj, s);
       RF_HIP(hipMemcpyAsync(hp + kMaxKrylov, proj, 8 * cols, hipMemcpyDeviceToHost, s));
       sync(op);
       for (int pass = 0; pass < 2; ++pass) {
@@ -972,9 +974,9 @@ int krylov_impl(rfhip_op *op, const double *v_host, double t, int max_dim, doubl
   return dim;
 }
 
-// ---- adaptive Krylov exponential ------------------------------------------
+// ---- Krylov exponentials on a DCGS2 basis ---------------------------------
 //
-// The adaptive exponential's Arnoldi basis, built one column at a time by
+// The exponentials' Arnoldi basis, built one column at a time by
 // classical Gram-Schmidt with delayed reorthogonalisation (DCGS2,
 // Swirydowicz, Langou, Ananthan, Yang and Thomas, "Low synchronization
 // Gram-Schmidt and generalized minimal residual algorithms", 2021): column
@@ -1003,11 +1005,16 @@ struct Arnoldi {
   // compressed basis (RFHIP_KRYLOV_BASIS_COMPRESSED): the finished columns
   // as f32 hi [cap][n] + bf16 lo [cap][nl] in kb_cbasis; the provisional
   // vector (which starts as the state) and the product A q in kb_basis
-  bool cb = false;
+  bool cb;
   int64_t nl = 0;
 
-  Arnoldi(rfhip_op *o, int capacity) : op(o), n(nvec(o)), cap(capacity) {
-    cb = op->kb_mode == RFHIP_KRYLOV_BASIS_COMPRESSED;
+  // The ETD augmentation [[A, b], [0, 0]]: each vector carries a scalar
+  // component on the host (sc[c] of column c), which enters the products
+  // there; b is op->src.
+  bool aug = false;
+  std::vector<double> sc;
+
+  Arnoldi(rfhip_op *o, int capacity, bool compressed) : op(o), n(nvec(o)), cap(capacity), cb(compressed) {
     if (cb) {
       nl = (n + 1) & ~int64_t(1);
       op->kb_cbasis.alloc((size_t)cap * (4 * (size_t)n + 2 * (size_t)nl));
@@ -1025,6 +1032,7 @@ struct Arnoldi {
       op->k.alloc(4 * n);
     }
     H.assign((size_t)(cap + 1) * cap, 0.0);
+    sc.assign((size_t)cap + 2, 0.0);
   }
   double *basis() const { return op->kb_basis.as<double>(); }
   double *col(int c) const { return basis() + (int64_t)c * n; }
@@ -1059,22 +1067,26 @@ struct Arnoldi {
   }
   // Finishes v_j (j = cols) and starts q_{j+1}; at j = 0 sets beta = |q_0|.
   // A breakdown (|q_j - V_j s| below the threshold of propagator.rs) leaves
-  // cols = j, H[j][j-1] = 0 and broke set.
-  void extend() {
+  // cols = j, H[j][j-1] = 0 and broke set. Returns false, with H as it was,
+  // on a non-finite product.
+  bool extend() {
     RF_REQUIRE(pending && !broke && cols < cap, "adaptive Arnoldi: no provisional column to extend");
     hipStream_t s = op->stream;
     const int j = cols;
     double *dev = op->kb_proj.as<double>(), *hp = op->kb_host.as<double>(), *part = op->kb_part.as<double>();
     apply(qv(j), zv(j));
+    if (aug && sc[j] != 0.0) launch_axpy(zv(j), op->src.as<double>(), sc[j], n, s);
     if (cb)
       launch_gram2c(chi(), clo(), n, nl, j, qv(j), zv(j), part, nblk, dev + kGram, s);
     else
       launch_gram2(basis(), n, j + 2, part, nblk, dev + kGram, s);
     RF_HIP(hipMemcpyAsync(hp + kGram, dev + kGram, 8 * (size_t)(2 * (j + 1)), hipMemcpyDeviceToHost, s));
     sync(op);
-    const double *g = hp + kGram;  // g[2c] = b_c . q_j, g[2c + 1] = b_c . z
+    double *g = hp + kGram;  // g[2c] = b_c . q_j, g[2c + 1] = b_c . z (whose scalar component is 0)
+    if (aug)
+      for (int c = 0; c <= j; ++c) g[2 * c] += sc[c] * sc[j];
     const double alpha = g[2 * j], gamma = g[2 * j + 1];
-    RF_REQUIRE(std::isfinite(alpha) && std::isfinite(gamma), "adaptive Arnoldi: non-finite basis vector");
+    if (!std::isfinite(alpha) || !std::isfinite(gamma)) return false;
     double r2 = alpha, sp = 0.0;
     for (int c = 0; c < j; ++c) {
       r2 -= g[2 * c] * g[2 * c];
@@ -1086,7 +1098,7 @@ struct Arnoldi {
       if (beta == 0.0) {
         broke = true;
         pending = false;
-        return;
+        return true;
       }
     } else {
       for (int c = 0; c < j; ++c) h(c, j - 1) += g[2 * c];
@@ -1094,7 +1106,7 @@ struct Arnoldi {
         h(j, j - 1) = 0.0;
         broke = true;
         pending = false;
-        return;
+        return true;
       }
       h(j, j - 1) = r;
     }
@@ -1113,6 +1125,15 @@ struct Arnoldi {
     }
     cf[2 * j] = cv[j] / r;
     cf[2 * j + 1] = 1.0 / r;
+    if (aug) {
+      double qs = sc[j], zs = -cf[2 * j] * sc[j];
+      for (int c = 0; c < j; ++c) {
+        qs -= cf[c] * sc[c];
+        zs -= cf[j + c] * sc[c];
+      }
+      sc[j] = qs / r;
+      sc[j + 1] = zs / r;
+    }
     RF_HIP(hipMemcpyAsync(dev + kCoef, cf, 8 * (size_t)(2 * j + 2), hipMemcpyHostToDevice, s));
     if (cb)
       launch_dcgs_updatec(chi(), clo(), n, nl, j, dev + kCoef, qv(j), zv(j), part, nblk, dev + kNorm, s);
@@ -1120,13 +1141,14 @@ struct Arnoldi {
       launch_dcgs_update(basis(), n, j, dev + kCoef, part, nblk, dev + kNorm, s);
     RF_HIP(hipMemcpyAsync(hp + kNorm, dev + kNorm, 8, hipMemcpyDeviceToHost, s));
     cols = j + 1;
+    return true;
   }
   // H[cols][cols-1] from |q_cols| (the first-pass residual norm), for the
   // proposer's features before the column is finished.
   void provisional() {
     if (!pending || broke || cols == 0) return;
     sync(op);
-    h(cols, cols - 1) = std::sqrt(std::max(op->kb_host.as<double>()[kNorm], 0.0));
+    h(cols, cols - 1) = std::sqrt(std::max(op->kb_host.as<double>()[kNorm], 0.0) + sc[cols] * sc[cols]);
   }
   // Reorthogonalises the last provisional vector: closes column cols-1 of H
   // (its correction and H[cols][cols-1]); a breakdown sets broke.
@@ -1149,6 +1171,8 @@ struct Arnoldi {
       RF_HIP(hipMemcpyAsync(hp + kGram, dev + kGram, 8 * (size_t)(j + 1), hipMemcpyDeviceToHost, s));
       sync(op);
     }
+    if (aug)
+      for (int c = 0; c <= j; ++c) hp[kGram + c] += sc[c] * sc[j];
     double r2 = hp[kGram + j];
     for (int c = 0; c < j; ++c) {
       h(c, j - 1) += hp[kGram + c];
@@ -1183,6 +1207,86 @@ struct Arnoldi {
   }
 };
 
+// exp(tA) v (aug: the ETD step, [[A, b], [0, 0]] with b = op->src) on one
+// basis of at most max_dim columns, ended by a breakdown or by the
+// a-posteriori estimate below tol (propagator.rs:278-294). Bound by the reads
+// of the basis: per column DCGS2 moves 2j + 6 vectors where CGS2 with its two
+// middle sweeps fused moved 3j + 7 (201,600 tets at N = 3, 26 columns: 49 ms a
+// call against 68).
+// The estimate is taken from the provisional column first, which differs
+// from the closed one by rounding only; the reorthogonalisation that closes
+// it runs where that passes, so the last column costs no apply of its own.
+int krylov_impl(rfhip_op *op, const double *v_host, double t, int max_dim, double tol, bool aug, double *out) {
+  const int64_t n = nvec(op);
+  RF_REQUIRE(max_dim >= 1 && max_dim <= kMaxKrylov, "Krylov dimension must be in [1, 64]");
+  hipStream_t s = op->stream;
+  Arnoldi ar(op, max_dim, false);
+  op->kb_x.alloc(8 * n);
+  op->kb_out.alloc(8 * n);
+  h2d_layout_f64(op, v_host, op->kb_x.as<double>());
+  sync(op);
+  const auto t_begin = std::chrono::steady_clock::now();
+  double *hp = op->kb_host.as<double>(), *dev = op->kb_proj.as<double>();
+  launch_multi_dot(op->kb_x.as<double>(), n, 1, op->kb_x.as<double>(), op->kb_part.as<double>(), ar.nblk, dev, s);
+  RF_HIP(hipMemcpyAsync(hp, dev, 8, hipMemcpyDeviceToHost, s));
+  sync(op);
+  const double beta = std::sqrt(hp[0] + (aug ? 1.0 : 0.0));
+  if (beta == 0.0) {
+    std::fill(out, out + op->n_dof, 0.0);
+    op->last_call_ms = 0.0;
+    return 0;
+  }
+  if (!std::isfinite(beta)) return krylov_cgs2(op, v_host, t, max_dim, tol, aug, out);
+  // Normalised first: an FP32 operator's apply takes any scale of v.
+  launch_scale(op->kb_x.as<double>(), ar.state(), n, 1.0 / beta, s);
+  ar.begin();
+  ar.aug = aug;
+  ar.sc[0] = aug ? 1.0 / beta : 0.0;
+  std::vector<double> th, eth;
+  auto hess_exp = [&](int d) {
+    th.assign((size_t)d * d, 0.0);
+    eth.assign((size_t)d * d, 0.0);
+    for (int a = 0; a < d; ++a)
+      for (int b = 0; b < d; ++b) th[(size_t)a * d + b] = t * ar.h(a, b);
+    expm_host(th.data(), d, eth.data());
+  };
+  auto estimate = [&](int d) {
+    hess_exp(d);
+    return ar.h(d, d - 1) * std::fabs(eth[(size_t)(d - 1) * d]);
+  };
+  std::vector<double> column(max_dim + 1);
+  bool have_exp = false;
+  for (;;) {
+    if (!ar.extend()) return krylov_cgs2(op, v_host, t, max_dim, tol, aug, out);
+    const int d = ar.cols;
+    if (ar.broke) break;
+    if (d == max_dim) {
+      ar.finalize();
+      break;
+    }
+    if (!(tol > 0.0)) continue;
+    ar.provisional();
+    if (ar.h(d, d - 1) >= kArnoldiBreakdown && !(estimate(d) < 1.0001 * tol)) continue;
+    for (int c = 0; c <= d; ++c) column[c] = ar.h(c, d - 1);
+    ar.finalize();
+    if (ar.broke || (have_exp = estimate(d) < tol)) break;
+    for (int c = 0; c <= d; ++c) ar.h(c, d - 1) = column[c];
+    ar.pending = true;
+  }
+  const int dim = ar.cols;
+  for (int a = 0; a < dim; ++a)
+    for (int b = 0; b < dim; ++b)
+      if (!std::isfinite(ar.h(a, b))) return krylov_cgs2(op, v_host, t, max_dim, tol, aug, out);
+  if (!have_exp) hess_exp(dim);
+  for (int i = 0; i < dim; ++i) hp[Arnoldi::kCoef + i] = beta * ar.beta * eth[(size_t)i * dim];
+  RF_HIP(hipMemcpyAsync(dev + Arnoldi::kCoef, hp + Arnoldi::kCoef, 8 * (size_t)dim, hipMemcpyHostToDevice, s));
+  launch_lincomb(ar.basis(), n, dim, dev + Arnoldi::kCoef, op->kb_out.as<double>(), s);
+  sync(op);
+  op->last_call_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_begin).count();
+  d2h_layout_f64(op, op->kb_out.as<double>(), out);
+  return dim;
+}
+
 // exp(t_end A) v with a step size and Krylov dimension chosen per step: the
 // plain error-controlled controller, or the network's proposals: its m sets
 // the basis and its h seeds a search for the largest step the same
@@ -1190,7 +1294,7 @@ struct Arnoldi {
 void adaptive_impl(rfhip_op *op, const double *v_host, double t_end, const rfhip_expctl &ctl, rfhip_mlp *mlp,
                    rfhip_exp_step *log, int64_t log_cap, double *hess, int hess_dim, int64_t *n_steps, double *out) {
   const int cap = std::max(ctl.m, ctl.m_max);
-  Arnoldi ar(op, cap);
+  Arnoldi ar(op, cap, op->kb_mode == RFHIP_KRYLOV_BASIS_COMPRESSED);
   double *x = ar.state();
   h2d_layout_f64(op, v_host, x);
   sync(op);
@@ -1203,11 +1307,11 @@ void adaptive_impl(rfhip_op *op, const double *v_host, double t_end, const rfhip
     RF_REQUIRE(nst < ctl.max_steps, "adaptive exponential: more than max_steps steps");
     const auto t_step = std::chrono::steady_clock::now();
     ar.begin();
-    ar.extend();
+    RF_REQUIRE(ar.extend(), "adaptive Arnoldi: non-finite basis vector");
     if (ar.beta == 0.0) break;  // a zero state stays zero
     if (nst == 0) rate = ctl.tol * ar.beta / t_end;
     const double t_left = t_end - t;
-    if (!ar.broke) ar.extend();
+    if (!ar.broke) RF_REQUIRE(ar.extend(), "adaptive Arnoldi: non-finite basis vector");
     ar.provisional();
     rfhip_exp_step rec{};
     rec.t = t;
@@ -1238,7 +1342,7 @@ void adaptive_impl(rfhip_op *op, const double *v_host, double t_end, const rfhip
       h_prop = h_next > 0.0 ? std::min(h_next, t_left) : 0.0;
       m_prop = ctl.m;
     }
-    while (!ar.broke && ar.cols < m_prop) ar.extend();
+    while (!ar.broke && ar.cols < m_prop) RF_REQUIRE(ar.extend(), "adaptive Arnoldi: non-finite basis vector");
     ar.finalize();
     const int d = ar.cols;
     rec.m = d;

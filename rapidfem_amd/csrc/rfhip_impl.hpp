@@ -405,11 +405,6 @@ void launch_dcgs_updatec(float *hi, uint16_t *lo, int64_t n, int64_t nl, int j, 
                          const double *z, double *partials, int nblk, double *norm2, hipStream_t s);
 void launch_lincombc(const float *hi, const uint16_t *lo, int64_t n, int64_t nl, int dim, const double *coef,
                      double *out, hipStream_t s);
-// w -= basis[:, :cols] proj, then proj_out = basis[:, :cols]^T w (the updated
-// w): a CGS2 first-pass update fused with the second pass's projections.
-// proj_out may be proj: it is written after every block has read proj.
-void launch_axpy_dot(double *w, const double *basis, int64_t n, int cols, const double *proj, double *partials,
-                     int nblk, double *proj_out, hipStream_t s);
 void launch_scale(const double *w, double *dst, int64_t n, double inv, hipStream_t s);
 void launch_lincomb(const double *basis, int64_t n, int dim, const double *coef, double *out, hipStream_t s);
 void launch_axpy(double *w, const double *x, double a, int64_t n, hipStream_t s);

@@ -227,9 +227,6 @@ constexpr int kMaxCols = 64;
 // once. The streaming updates take their columns eight at a time.
 constexpr int kDotTile = 8;
 constexpr int kDotTileM = 16;
-// Largest column count k_axpy_dot holds in registers; above it the update
-// and the products run as two sweeps.
-constexpr int kAxpyDotMaxCols = 48;
 // Per-block partial dot products of w with basis columns 0..cols-1, kDotTileM
 // columns per sweep over the block's contiguous range. With VEC (n even, so
 // every column starts 16-byte aligned) each lane reads two consecutive
@@ -328,56 +325,7 @@ __global__ void __launch_bounds__(kBS) k_axpy_basis_norm(double *__restrict__ w,
   const double t = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
-// The first pass's update and the second pass's projections of classical
-// Gram-Schmidt with reorthogonalisation in one sweep over the basis:
-// w -= sum_c proj[c] basis_c, then the per-block partials of basis_c . w
-// (the updated w) over contiguous per-block slices as in k_multi_dot. Each
-// lane keeps its entry of every column in registers between the update and
-// the products, so the basis is read once instead of twice.
-// MAXC >= cols is a multiple of 4 and the body has no branch per column:
-// columns cols..MAXC-1 reload column cols-1 (a cache hit) with coefficient
-// 0, so every load issues before the first use and the waits count down.
-template <int MAXC>
-__global__ void __launch_bounds__(kBS) k_axpy_dot(double *__restrict__ w, const double *__restrict__ basis,
-                                                  int64_t n, int cols, const double *__restrict__ proj,
-                                                  double *__restrict__ part) {
-  __shared__ double sh[kBS / 64];
-  __shared__ double sp[MAXC];
-  for (int c = threadIdx.x; c < MAXC; c += kBS) sp[c] = c < cols ? proj[c] : 0.0;
-  __syncthreads();
-  const int64_t chunk = (n + gridDim.x - 1) / gridDim.x;
-  const int64_t i0 = (int64_t)blockIdx.x * chunk;
-  const int64_t i1 = i0 + chunk < n ? i0 + chunk : n;
-  double acc[MAXC];
-#pragma unroll
-  for (int c = 0; c < MAXC; ++c) acc[c] = 0.0;
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += kBS) {
-    double b[MAXC];
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) b[c] = basis[(int64_t)(c < cols ? c : cols - 1) * n + i];
-    double wi = w[i];
-    // z is 0 (i < n < 2^62) but depends on i, so the coefficients are read
-    // from LDS (a broadcast) at each use instead of being held in two VGPRs
-    // per column across the loop.
-    const int z = (int)(i >> 62);
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) wi -= sp[c + z] * b[c];
-    w[i] = wi;
-#pragma unroll
-    for (int c = 0; c < MAXC; ++c) acc[c] += b[c] * wi;
-  }
-  // A guard, not a break: with a constant trip count the loop unrolls fully
-  // and acc stays in registers (an early exit left it in scratch memory
-  // above 16 columns).
-#pragma unroll
-  for (int c = 0; c < MAXC; ++c) {
-    if (c < cols) {
-      const double t = block_sum(acc[c], sh);
-      if (threadIdx.x == 0) part[(int64_t)blockIdx.x * cols + c] = t;
-    }
-  }
-}
-// ---- CGS2 with delayed reorthogonalisation (the adaptive Arnoldi) --------
+// ---- CGS2 with delayed reorthogonalisation (Arnoldi, rfhip_api.hip) -------
 //
 // Per-block partials of the Gram products of basis columns 0..cols-1 with
 // the last two, b_{cols-2} and b_{cols-1} (the provisional vector q and the
@@ -968,7 +916,8 @@ int krylov_dot_blocks(int64_t n) { return (int)grid_for(n, 1024); }
 
 void launch_multi_dot(const double *basis, int64_t n, int cols, const double *w, double *partials, int nblk,
                       double *proj, hipStream_t s) {
-  RF_REQUIRE(cols <= kMaxCols, "Krylov dimension above 64");
+  // a basis of 64 columns closes its last one against the provisional vector
+  RF_REQUIRE(cols <= kMaxCols + 1, "Krylov dimension above 64");
   if (n % 2 == 0)
     hipLaunchKernelGGL(k_multi_dot<true>, dim3(nblk), dim3(kBS), 0, s, basis, n, cols, w, partials);
   else
@@ -986,30 +935,9 @@ void launch_axpy_basis_norm(double *w, const double *basis, int64_t n, int cols,
   hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(kBS), 0, s, partials, nblk, norm2);
   RF_HIP(hipGetLastError());
 }
-void launch_axpy_dot(double *w, const double *basis, int64_t n, int cols, const double *proj, double *partials,
-                     int nblk, double *proj_out, hipStream_t s) {
-  RF_REQUIRE(cols >= 1 && cols <= kMaxCols, "Krylov dimension above 64");
-  if (cols > kAxpyDotMaxCols) {
-    launch_axpy_basis_norm(w, basis, n, cols, proj, partials, nblk, proj_out, s);
-    launch_multi_dot(basis, n, cols, w, partials, nblk, proj_out, s);
-    return;
-  }
-  const dim3 g(nblk), b(kBS);
-  switch ((cols + 3) / 4) {
-#define RF_AXPY_DOT(q)                                                                          \
-  case q:                                                                                       \
-    hipLaunchKernelGGL(k_axpy_dot<4 * q>, g, b, 0, s, w, basis, n, cols, proj, partials);       \
-    break;
-    RF_AXPY_DOT(1) RF_AXPY_DOT(2) RF_AXPY_DOT(3) RF_AXPY_DOT(4) RF_AXPY_DOT(5) RF_AXPY_DOT(6)
-    RF_AXPY_DOT(7) RF_AXPY_DOT(8) RF_AXPY_DOT(9) RF_AXPY_DOT(10) RF_AXPY_DOT(11) RF_AXPY_DOT(12)
-#undef RF_AXPY_DOT
-  }
-  hipLaunchKernelGGL(k_dot_finish, dim3(cols), dim3(kBS), 0, s, partials, nblk, cols, proj_out);
-  RF_HIP(hipGetLastError());
-}
 void launch_gram2(const double *basis, int64_t n, int cols, double *partials, int nblk, double *out,
                   hipStream_t s) {
-  RF_REQUIRE(cols >= 2 && cols <= kMaxCols, "Krylov dimension above 64");
+  RF_REQUIRE(cols >= 2 && cols <= kMaxCols + 1, "Krylov dimension above 64");
   if (n % 2 == 0)
     hipLaunchKernelGGL(k_gram2<true>, dim3(nblk), dim3(kBS), 0, s, basis, n, cols, partials);
   else
@@ -1019,7 +947,7 @@ void launch_gram2(const double *basis, int64_t n, int cols, double *partials, in
 }
 void launch_dcgs_update(double *basis, int64_t n, int j, const double *coef, double *partials, int nblk,
                         double *norm2, hipStream_t s) {
-  RF_REQUIRE(j >= 0 && j + 1 < kMaxCols, "Krylov dimension above 64");
+  RF_REQUIRE(j >= 0 && j < kMaxCols, "Krylov dimension above 64");
   if (n % 2 == 0)
     hipLaunchKernelGGL(k_dcgs_update<true>, dim3(nblk), dim3(kBS), 0, s, basis, n, j, coef, partials);
   else
