@@ -167,9 +167,9 @@ void build_plain(rfhip_op *op, const rfhip_op_desc &d) {
 }
 // Stage-kernel variant an operator starts with: k_quad (variant 9) where its
 // tables exist, the fastest on MI355X at every order and both register layouts
-// from 48 tets to the largest meshes swept. us per stage, fastest other variant
+// but for the ranges named below. us per stage, fastest other variant
 // against k_quad, N = 1..4: FP64 registers, 1,296 tets 5.6 / 3.9, 7.6 / 5.4,
-// 9.4 / 8.4, 15.4 / 15.1; 1.3M / 768k / 324k / 384k tets 288 / 262, 484 / 350,
+// 9.4 / 8.4, 15.4 / 15.1; 1.3M / 768k / 324k / 384k tets 288 / 271, 484 / 350,
 // 416 / 290, 1232 / 690; compressed registers, the same large meshes 235 / 221,
 // 410 / 306, 376 / 262, 1170 / 735, with the same bits as the variants named
 // below (their rounding of p to f32 turns any other order of the sums into
