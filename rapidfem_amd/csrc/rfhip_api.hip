@@ -176,16 +176,17 @@ void build_plain(rfhip_op *op, const rfhip_op_desc &d) {
 // differences of its own size within a few dozen stages). Compressed registers
 // on small meshes at N = 3, 4, where a stage is one group's chain of operations
 // and that order makes it longer, stay with those variants (1,296 tets: 9.6 /
-// 9.9 and 16.6 / 19.2 us; 3,072: 10.2 / 10.2 and 20.5 / 19.0), and so do they at
-// N = 1 between the size where every group runs at once and the one where the
-// state no longer fits the 256 MB cache (17,640 tets 9.0 / 7.6, 27,648 8.2 / 8.8,
-// 196,608 33 / 36, 384,000 61 / 67, 750,000 139 / 125). Operators without
+// 10.0 and 16.7 / 19.6 us; 2,688: 10.1 / 10.3 and 19.4 / 19.3; 3,072: 10.3 / 10.3
+// and 20.8 / 19.4; 6,000: 14.0 / 11.6 and 33.0 / 22.1), and so do they at N = 1
+// in a range that the sweep shows and nothing yet explains: 24,576 tets 8.0 /
+// 7.8, 26,112 8.1 / 8.8, 31,212 8.4 / 8.9, 45,600 13.2 / 14.0, 66,792 15.1 /
+// 15.5, then 101,400 22.5 / 21.6. Operators without
 // the tables (no permuted node tables, or a state of 2^32 bytes and more) start
 // with the fastest of the rest. autotune re-picks on the operator's own mesh.
 int default_variant(int order, int form, const StageArgs &a) {
   if (form_vmf(form)) return 1;
   const bool c = form == RFHIP_FORM_FUSED_F64C;
-  const bool keep = c && (order >= 3 ? a.n_elem < 2560 : order == 1 && a.n_elem > 24576 && a.n_elem < 700000);
+  const bool keep = c && (order == 1 ? a.n_elem > 24576 && a.n_elem < 70000 : order == 3 ? a.n_elem < 3200 : order == 4 && a.n_elem < 2560);
   if (!keep && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
   switch (order) {
     case 1: return c ? 7 : 5;
@@ -526,8 +527,9 @@ void rhs_into(rfhip_op *op, const void *x, void *k, int kind, int64_t dof, doubl
 // pair around each dominant-kernel launch. dev_wave: the drive is the
 // device-assembled port source held at the waveform sample
 // op->gseq[*op->gctr] (kind/dof/g unused), and the step advances *op->gctr.
+// beside: StageArgs.
 void lserk_step(rfhip_op *op, double h, int kind, int64_t dof, double g, hipEvent_t *stage_ev,
-                bool dev_wave = false) {
+                bool dev_wave = false, int64_t beside = 0) {
   hipStream_t s = op->stream;
   if (dev_wave) kind = RFHIP_DRIVE_FREE;
   for (int st = 0; st < 5; ++st) {
@@ -542,6 +544,7 @@ void lserk_step(rfhip_op *op, double h, int kind, int64_t dof, double g, hipEven
       a.sa = kLsA[st];
       a.sb = kLsB[st];
       a.dt = h;
+      a.beside = beside;
       fill_source(op, a, kind, dof, g);
       launch_stage(op->order, op->form, 1, a, s);
       if (stage_ev) RF_HIP(hipEventRecord(stage_ev[2 * st + 1], s));
@@ -1446,9 +1449,16 @@ void batch_lserk_impl(rfhip_op *const *ops, int32_t n_ops, const double *dt, int
     for (auto e : ev)
       if (e) (void)hipEventDestroy(e);
   };
+  // what the stages of each operator, and of all, touch over and over: y twice
+  // and p (form_compressed: 16 bytes a value) and the geometry
+  auto reg_bytes = [&](int32_t i) {
+    return (form_compressed(ops[i]->form) ? 16 : 24) * nvec(ops[i]) + 92 * ops[i]->n_elem;
+  };
+  int64_t all_bytes = 0;
+  for (int32_t i = 0; i < n_ops; ++i) all_bytes += reg_bytes(i);
   auto step_all = [&] {
     for (int32_t i = 0; i < n_ops; ++i)
-      lserk_step(ops[i], dt[i], RFHIP_DRIVE_FREE, 0, 0.0, nullptr, driven[(size_t)i] != 0);
+      lserk_step(ops[i], dt[i], RFHIP_DRIVE_FREE, 0, 0.0, nullptr, driven[(size_t)i] != 0, all_bytes - reg_bytes(i));
   };
   try {
     for (auto &e : ev) RF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));

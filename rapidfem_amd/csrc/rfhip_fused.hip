@@ -2613,7 +2613,7 @@ bool kcl_stage_fusable(int form, const StageArgs &a) { return !form_vmf(form) &&
 
 int64_t kcl_stage_slots(int order, const StageArgs &a, bool r64) {
   if (a.variant == kQuadVariant && a.quad)
-    return quad_kcl_slots((order + 1) * (order + 2) * (order + 3) / 6, r64, a.n_elem);
+    return quad_kcl_slots((order + 1) * (order + 2) * (order + 3) / 6, r64, a);
   switch ((order + 1) * (order + 2) * (order + 3) / 6) {
     case 4: return kcl_grid<4>(a, r64) * (kFusedWG / 64);
     case 10: return kcl_grid<10>(a, r64) * (kFusedWG / 64);

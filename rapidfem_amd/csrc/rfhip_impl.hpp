@@ -140,6 +140,7 @@ struct DevOp {
 // Vectors use the reference's AoS layout y[(e*Np + node)*6 + comp].
 struct StageArgs {
   int64_t n_elem;
+  int64_t beside;         // bytes of the registers of operators stepped beside this one (k_quad's cache hints)
   double alpha;
   int variant;            // kernel variant (rfhip_fused.hip)
   const double *dT;       // 3*Np*Np: dT[(k*Np + j)*Np + i] = D_k[i][j]
@@ -308,7 +309,7 @@ bool clane_pack(int np, const int *face_nodes, const double *const D[3], const d
 // sums its last KCL stage leaves in a.kpart.
 bool quad_pack(int np, const double *const D[3], const double *lift, bool seq, std::vector<double> &out);
 void launch_quad(int np, int epi, const StageArgs &a, hipStream_t s);
-int64_t quad_kcl_slots(int np, bool r64, int64_t n_elem);
+int64_t quad_kcl_slots(int np, bool r64, const StageArgs &a);
 // Debye block after an applied derivative (dy = A y; f32: plain FP32 form),
 // with the drive of the P rows, and after a fused LSERK4 stage
 // (rfhip_debye.hip). No-ops without Debye elements.

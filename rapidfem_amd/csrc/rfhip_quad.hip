@@ -281,26 +281,31 @@ template <class T>
 __device__ __forceinline__ T ld_al(const void *p, uint32_t byte) {
   return *reinterpret_cast<const T *>(static_cast<const char *>(p) + byte);
 }
-// Streamed accesses: the update's registers and every store are touched once
-// per launch and are kept from displacing the state that neighbours gather.
-template <class T>
-__device__ __forceinline__ T ld_nt(const void *p, uint32_t byte) {
-  typedef unsigned W __attribute__((ext_vector_type(sizeof(T) / 4)));
-  return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const W *>(static_cast<const char *>(p) + byte)));
+// Accesses of the update's registers and of every result, each touched once
+// per launch. NT: streamed, kept from displacing the state that neighbours
+// gather (quad_streams below says when).
+template <bool NT, class T>
+__device__ __forceinline__ T ld_reg(const void *p, uint32_t byte) {
+  if constexpr (NT) {
+    typedef unsigned W __attribute__((ext_vector_type(sizeof(T) / 4)));
+    return __builtin_bit_cast(T, __builtin_nontemporal_load(reinterpret_cast<const W *>(static_cast<const char *>(p) + byte)));
+  } else {
+    return ld_al<T>(p, byte);
+  }
 }
-template <class T>
-__device__ __forceinline__ void st_al(void *p, uint32_t byte, T v) {
-  typedef unsigned W __attribute__((ext_vector_type(sizeof(T) / 4)));
-  __builtin_nontemporal_store(__builtin_bit_cast(W, v), reinterpret_cast<W *>(static_cast<char *>(p) + byte));
+template <bool NT, class T>
+__device__ __forceinline__ void st_reg(void *p, uint32_t byte, T v) {
+  if constexpr (NT) {
+    typedef unsigned W __attribute__((ext_vector_type(sizeof(T) / 4)));
+    __builtin_nontemporal_store(__builtin_bit_cast(W, v), reinterpret_cast<W *>(static_cast<char *>(p) + byte));
+  } else {
+    *reinterpret_cast<T *>(static_cast<char *>(p) + byte) = v;
+  }
 }
 
 template <bool CIN, int VW, bool NT = false>
 __device__ __forceinline__ Lin<CIN, VW> load_lin(const void *hi, const void *lo, uint32_t i) {
-  auto get = [](auto z, const void *p, uint32_t byte) {
-    using V = decltype(z);
-    if constexpr (NT) return ld_nt<V>(p, byte);
-    else return ld_al<V>(p, byte);
-  };
+  auto get = [](auto z, const void *p, uint32_t byte) { return ld_reg<NT, decltype(z)>(p, byte); };
   Lin<CIN, VW> r;
   if constexpr (CIN && VW == 4) {
     r.h = get(float4{}, hi, 4 * i);
@@ -333,7 +338,7 @@ __device__ __forceinline__ void lin_f64(const Lin<CIN, VW> &r, double *v) {
   }
 }
 // VW FP64 values stored as f32 hi + bf16 lo.
-template <int VW>
+template <bool NT, int VW>
 __device__ __forceinline__ void store_c(void *hi, void *lo, uint32_t i, const double *v) {
   float h[VW], r[VW];
 #pragma unroll
@@ -342,69 +347,69 @@ __device__ __forceinline__ void store_c(void *hi, void *lo, uint32_t i, const do
     r[q] = (float)(v[q] - (double)h[q]);
   }
   if constexpr (VW == 4) {
-    st_al(hi, 4 * i, make_float4(h[0], h[1], h[2], h[3]));
-    st_al(lo, 2 * i, make_uint2(bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3])));
+    st_reg<NT>(hi, 4 * i, make_float4(h[0], h[1], h[2], h[3]));
+    st_reg<NT>(lo, 2 * i, make_uint2(bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3])));
   } else {
-    st_al(hi, 4 * i, make_float2(h[0], h[1]));
-    st_al(lo, 2 * i, bf16_pair(r[0], r[1]));
+    st_reg<NT>(hi, 4 * i, make_float2(h[0], h[1]));
+    st_reg<NT>(lo, 2 * i, bf16_pair(r[0], r[1]));
   }
 }
-template <int VW>
+template <bool NT, int VW>
 __device__ __forceinline__ void store_d(void *p, uint32_t i, const double *v) {
 #pragma unroll
-  for (int q = 0; q < VW / 2; ++q) st_al(p, 8 * i + 16 * q, make_double2(v[2 * q], v[2 * q + 1]));
+  for (int q = 0; q < VW / 2; ++q) st_reg<NT>(p, 8 * i + 16 * q, make_double2(v[2 * q], v[2 * q + 1]));
 }
-template <int VW>
+template <bool NT, int VW>
 __device__ __forceinline__ void store_f(void *p, uint32_t i, const float *v) {
   if constexpr (VW == 4)
-    st_al(p, 4 * i, make_float4(v[0], v[1], v[2], v[3]));
+    st_reg<NT>(p, 4 * i, make_float4(v[0], v[1], v[2], v[3]));
   else
-    st_al(p, 4 * i, make_float2(v[0], v[1]));
+    st_reg<NT>(p, 4 * i, make_float2(v[0], v[1]));
 }
 template <int VW>
 struct Flt {
   float v[VW];
 };
-template <int VW>
+template <bool NT, int VW>
 __device__ __forceinline__ Flt<VW> load_f(const void *p, uint32_t i) {
   if constexpr (VW == 4) {
-    const float4 t = ld_nt<float4>(p, 4 * i);
+    const float4 t = ld_reg<NT, float4>(p, 4 * i);
     return {{t.x, t.y, t.z, t.w}};
   } else {
-    const float2 t = ld_nt<float2>(p, 4 * i);
+    const float2 t = ld_reg<NT, float2>(p, 4 * i);
     return {{t.x, t.y}};
   }
 }
 
 // The linear registers an epilogue reads besides the state: p (LSERK4) or y
 // and err (KCL).
-template <int EPI, int VW>
+template <int EPI, int VW, bool NT>
 struct Upd {};
-template <int VW>
-struct Upd<1, VW> {
+template <int VW, bool NT>
+struct Upd<1, VW, NT> {
   Lin<false, VW> p;
-  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) { p = load_lin<false, VW, true>(io.p, nullptr, i); }
+  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) { p = load_lin<false, VW, NT>(io.p, nullptr, i); }
 };
-template <int VW>
-struct Upd<2, VW> {
+template <int VW, bool NT>
+struct Upd<2, VW, NT> {
   Flt<VW> p;
-  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) { p = load_f<VW>(io.p, i); }
+  __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) { p = load_f<NT, VW>(io.p, i); }
 };
-template <int VW>
-struct Upd<3, VW> {
+template <int VW, bool NT>
+struct Upd<3, VW, NT> {
   Lin<true, VW> y;
   Flt<VW> e;
   __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) {
-    y = load_lin<true, VW, true>(io.ky, io.ky_lo, i);
-    e = load_f<VW>(io.kerr, i);
+    y = load_lin<true, VW, NT>(io.ky, io.ky_lo, i);
+    e = load_f<NT, VW>(io.kerr, i);
   }
 };
-template <int VW>
-struct Upd<4, VW> {
+template <int VW, bool NT>
+struct Upd<4, VW, NT> {
   Lin<false, VW> y, e;
   __device__ __forceinline__ void load(const StageArgs &io, uint32_t i) {
-    y = load_lin<false, VW, true>(io.kyd, nullptr, i);
-    e = load_lin<false, VW, true>(io.kerrd, nullptr, i);
+    y = load_lin<false, VW, NT>(io.kyd, nullptr, i);
+    e = load_lin<false, VW, NT>(io.kerrd, nullptr, i);
   }
 };
 
@@ -415,10 +420,9 @@ __device__ __forceinline__ int64_t quad_block() {
 
 // Waves per SIMD the registers are fitted to: the most that leave no spills
 // (N = 2: 300 us at 3 waves, 342 at 2 with compressed registers; 427 at 3 with
-// 13 spilled, 350 at 2, with FP64 ones; N = 3 at 3 waves spills 48 to 100).
-// N = 1 takes 4 although 3 stream a large mesh faster (262 us against 271 for
-// 1.3M tets): up to 32,768 tets every group then runs at once (27,030 tets: 9.8
-// us per stage against 11.4).
+// 13 spilled, 350 at 2, with FP64 ones; N = 3 at 3 waves spills 48 to 100). At
+// N = 1 the LSERK4 stage runs 4 waves fitted to 3 or to 4 (116 to 122 VGPRs),
+// within 1 % of each other from 384 to 1.3M tets.
 template <int NP, int EPI>
 struct QuadWaves {
   static constexpr int v = NP == 4 ? (EPI <= 2 ? 4 : 3) : NP == 10 && (EPI == 0 || EPI == 2) ? 3 : 2;
@@ -426,14 +430,14 @@ struct QuadWaves {
 
 // EPI as in the other stage kernels: 0 apply, 1 LSERK4 stage with FP64
 // registers, 2 with compressed ones, 3 / 4 KCL stage with compressed / FP64
-// registers. CIN: the input state is f32 + bf16. nw: the waves of a block that
-// take groups (all of them load the tables).
-template <int NP, bool CIN, int EPI>
+// registers. CIN: the input state is f32 + bf16. NT: quad_streams. nw: the
+// waves of a block that take groups (all of them load the tables).
+template <int NP, bool CIN, int EPI, bool NT>
 __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_waves_per_eu(QuadWaves<NP, EPI>::v))) k_quad(StageArgs io, int nw) {
   using T = QuadTab<NP>;
   constexpr bool SEQ = CIN;
   using Z = QuadSize<NP, SEQ>;
-  constexpr int NG = T::NG, NT = T::NWB * 64, NFP = ElemTab<NP>::NFP;
+  constexpr int NG = T::NG, NTH = T::NWB * 64, NFP = ElemTab<NP>::NFP;
   constexpr int SE = 6 * NP;             // values per element
   constexpr int SW = kQuadEl * SE;       // values per group
   // Element stride in LDS, = 4 mod 8 in 8-byte banks: with the nodes of lanes
@@ -448,8 +452,8 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
   __shared__ __align__(16) uint4 snode[100];
   __shared__ int splace[2][4 * NG];  // LDS place in an element of column (0) and row (1) node (g, q)
   __shared__ __align__(16) double su_b[T::NWB][SZ + 8];  // + zeros the padding nodes read, + a place for what they write
-  for (int t = threadIdx.x; t < NFR * 16; t += NT) reinterpret_cast<double2 *>(sA)[t] = reinterpret_cast<const double2 *>(SEQ ? io.quad_seq : io.quad)[t];
-  for (int t = threadIdx.x; t < 100; t += NT) snode[t] = reinterpret_cast<const uint4 *>(io.quad_nodes)[t];
+  for (int t = threadIdx.x; t < NFR * 16; t += NTH) reinterpret_cast<double2 *>(sA)[t] = reinterpret_cast<const double2 *>(SEQ ? io.quad_seq : io.quad)[t];
+  for (int t = threadIdx.x; t < 100; t += NTH) snode[t] = reinterpret_cast<const uint4 *>(io.quad_nodes)[t];
   if ((int)threadIdx.x < 4 * NG) {
     const int g = threadIdx.x >> 2, r = threadIdx.x & 3;
     splace[1][threadIdx.x] = 6 * quad_row<NP, SEQ>(g, r);
@@ -670,7 +674,7 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
       nnmat = io.mat[e2];
     }
     constexpr bool kLateRegs = T::LATE || EPI == 4;
-    Upd<EPI, VW> up[EPI == 0 ? 1 : IT];
+    Upd<EPI, VW, NT> up[EPI == 0 ? 1 : IT];
     auto read_registers = [&] {
       if constexpr (EPI != 0) {
         const uint32_t last = gb + (uint32_t)(nel * SE - VW);
@@ -909,7 +913,7 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
             const double *kv = kr[k - k0];
             const uint32_t gi = gb + (uint32_t)i;
             if constexpr (EPI == 0) {
-              store_d<VW>(io.dy, gi, kv);
+              store_d<NT, VW>(io.dy, gi, kv);
             } else if constexpr (EPI == 1) {
               double po[VW], pn[VW], yn[VW];
               lin_f64<false, VW>(up[k].p, po);
@@ -918,8 +922,8 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
                 pn[c] = io.sa * po[c] + io.dt * kv[c];
                 yn[c] = yv[k][c] + io.sb * pn[c];
               }
-              store_d<VW>(io.p, gi, pn);
-              store_d<VW>(io.yout, gi, yn);
+              store_d<NT, VW>(io.p, gi, pn);
+              store_d<NT, VW>(io.yout, gi, yn);
             } else if constexpr (EPI == 2) {
               float pn[VW];
               double yn[VW];
@@ -932,8 +936,8 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
                 pn[c] = (float)v;
                 yn[c] = fma(io.sb, (double)pn[c], yv[k][c]);
               }
-              store_f<VW>(io.p, gi, pn);
-              store_c<VW>(io.yout, io.yout_lo, gi, yn);
+              store_f<NT, VW>(io.p, gi, pn);
+              store_c<NT, VW>(io.yout, io.yout_lo, gi, yn);
             } else if constexpr (EPI == 3) {
               // the arithmetic of node_kcl (rfhip_fused.hip)
               float en[VW];
@@ -949,12 +953,12 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
                 sn[c] = io.klast ? yn[c] : yn[c] + io.kamb * f;
                 if (io.klast) wsum += werr_term(bo[c], yn[c], er, io.katol, io.krtol);
               }
-              store_c<VW>(io.ky, io.ky_lo, gi, yn);
-              store_f<VW>(io.kerr, gi, en);
-              store_c<VW>(io.yout, io.yout_lo, gi, sn);
+              store_c<NT, VW>(io.ky, io.ky_lo, gi, yn);
+              store_f<NT, VW>(io.kerr, gi, en);
+              store_c<NT, VW>(io.yout, io.yout_lo, gi, sn);
               if (io.kfirst) {
-                st_al(io.kbak, 4 * gi, up[k].y.h);
-                st_al(io.kbak_lo, 2 * gi, up[k].y.l);
+                st_reg<NT>(io.kbak, 4 * gi, up[k].y.h);
+                st_reg<NT>(io.kbak_lo, 2 * gi, up[k].y.l);
               }
             } else {
               // the arithmetic of node_kcl64
@@ -970,10 +974,10 @@ __global__ void __launch_bounds__(QuadTab<NP>::NWB * 64) __attribute__((amdgpu_w
                 sn[c] = io.klast ? yn[c] : yn[c] + io.kamb * f;
                 if (io.klast) wsum += werr_term(bo[c], yn[c], er[c], io.katol, io.krtol);
               }
-              store_d<VW>(io.kyd, gi, yn);
-              store_d<VW>(io.kerrd, gi, er);
-              store_d<VW>(io.yout, gi, sn);
-              if (io.kfirst) store_d<VW>(io.kbakd, gi, yo);
+              store_d<NT, VW>(io.kyd, gi, yn);
+              store_d<NT, VW>(io.kerrd, gi, er);
+              store_d<NT, VW>(io.yout, gi, sn);
+              if (io.kfirst) store_d<NT, VW>(io.kbakd, gi, yo);
             }
           }
         }
@@ -1028,24 +1032,58 @@ struct QuadGrid {
   int64_t blocks;
   int waves;
 };
-template <int NP, bool CIN, int EPI>
+template <int NP, bool CIN, int EPI, bool NT>
 QuadGrid quad_grid(int64_t n_elem) {
   constexpr int NWB = QuadTab<NP>::NWB;
   const int64_t groups = (n_elem + kQuadEl - 1) / kQuadEl;
-  const Residency r = quad_resident(reinterpret_cast<const void *>(&k_quad<NP, CIN, EPI>), NWB * 64);
+  const Residency r = quad_resident(reinterpret_cast<const void *>(&k_quad<NP, CIN, EPI, NT>), NWB * 64);
   const int64_t nw = std::min<int64_t>(NWB, std::max<int64_t>(1, (groups + r.cus - 1) / r.cus));
   return {std::min((groups + nw - 1) / nw, r.cus * r.per_cu), (int)nw};
 }
-template <int NP, bool CIN, int EPI>
-void quad_launch(const StageArgs &a, hipStream_t s) {
-  const QuadGrid g = quad_grid<NP, CIN, EPI>(a.n_elem);
-  if (g.blocks > 0) hipLaunchKernelGGL((k_quad<NP, CIN, EPI>), dim3((unsigned)g.blocks), dim3(QuadTab<NP>::NWB * 64), 0,
+// Bytes of one value in the registers that an epilogue's launches alternate
+// between: state in and out and p, or state in and out, y, err and the backup.
+constexpr int quad_value_bytes(int epi) { return epi == 1 ? 24 : epi == 2 ? 16 : epi == 3 ? 28 : 40; }
+
+// Whether the registers are streamed. A step's launches return to the same
+// registers, and where those of this operator (with its geometry, 92 bytes an
+// element) and of what is stepped beside it fit the 256 MB last-level cache, a
+// streamed store sends out of it what the next launch reads. us per stage,
+// streamed / not, FP64 registers: N = 1, 196,608 tets (131 MB) 43.2 / 33.3 (the
+// fastest other variant 41.9), N = 4, 48,000 tets (246 MB) 100 / 98; above that
+// size what passes through should not displace the state: N = 1, 511,104 tets
+// (341 MB) 106 / 116, N = 3, 196,608 tets (584 MB) 175 / 189. Small registers
+// are faster streamed too: N = 1, 12,096 tets (8 MB) 6.3 / 6.9, N = 3, 6,000 tets
+// (18 MB) 10.8 / 11.5, then N = 1, 36,936 tets (25 MB) 14.4 / 12.3; compressed
+// ones 13.2 / 13.5 there (18 MB) and 22.8 / 22.1 at 101,400 tets (48 MB). The
+// apply (EPI 0) always streams: nothing returns to its result (the same within
+// 1 % up to 300 MB, 3 % faster above).
+bool quad_streams(int np, bool cin, int epi, const StageArgs &a) {
+  const int64_t mb = (int64_t)1 << 20;
+  const int64_t own = a.n_elem * (6 * np * quad_value_bytes(epi) + 92);
+  return epi == 0 || own < (cin ? 32 : 20) * mb || own + a.beside > 256 * mb;
+}
+template <int NP, bool CIN, int EPI, bool NT>
+void quad_launch_nt(const StageArgs &a, hipStream_t s) {
+  const QuadGrid g = quad_grid<NP, CIN, EPI, NT>(a.n_elem);
+  if (g.blocks > 0) hipLaunchKernelGGL((k_quad<NP, CIN, EPI, NT>), dim3((unsigned)g.blocks), dim3(QuadTab<NP>::NWB * 64), 0,
                        s, a, g.waves);
 }
-template <int NP>
-int64_t quad_slots(bool r64, int64_t n_elem) {
-  const QuadGrid g = r64 ? quad_grid<NP, false, 4>(n_elem) : quad_grid<NP, true, 3>(n_elem);
+template <int NP, bool CIN, int EPI>
+void quad_launch(const StageArgs &a, hipStream_t s) {
+  if (EPI == 0 || quad_streams(NP, CIN, EPI, a))
+    quad_launch_nt<NP, CIN, EPI, true>(a, s);
+  else
+    quad_launch_nt<NP, CIN, EPI, EPI == 0>(a, s);
+}
+template <int NP, bool CIN, int EPI>
+int64_t quad_slots_epi(const StageArgs &a) {
+  const QuadGrid g = quad_streams(NP, CIN, EPI, a) ? quad_grid<NP, CIN, EPI, true>(a.n_elem)
+                                                   : quad_grid<NP, CIN, EPI, false>(a.n_elem);
   return g.blocks * g.waves;
+}
+template <int NP>
+int64_t quad_slots(bool r64, const StageArgs &a) {
+  return r64 ? quad_slots_epi<NP, false, 4>(a) : quad_slots_epi<NP, true, 3>(a);
 }
 template <bool CIN, int EPI>
 void quad_orders(int np, const StageArgs &a, hipStream_t s) {
@@ -1130,12 +1168,12 @@ void launch_quad(int np, int epi, const StageArgs &a, hipStream_t s) {
   }
 }
 
-int64_t quad_kcl_slots(int np, bool r64, int64_t n_elem) {
+int64_t quad_kcl_slots(int np, bool r64, const StageArgs &a) {
   switch (np) {
-    case 4: return quad_slots<4>(r64, n_elem);
-    case 10: return quad_slots<10>(r64, n_elem);
-    case 20: return quad_slots<20>(r64, n_elem);
-    case 35: return quad_slots<35>(r64, n_elem);
+    case 4: return quad_slots<4>(r64, a);
+    case 10: return quad_slots<10>(r64, a);
+    case 20: return quad_slots<20>(r64, a);
+    case 35: return quad_slots<35>(r64, a);
     default: throw Error{RFHIP_EUNSUPPORTED, "the fused stage kernels run orders 1 to 4"};
   }
 }
