@@ -197,6 +197,20 @@ int default_variant(int order, int form, const StageArgs &a) {
   }
 }
 
+// Variant of the fused KCL stages (kcl_impl) where the LSERK4 stage's was not
+// pinned: the same but in two ranges of FP64 registers, where k_quad's KCL stage
+// is the slower one. At N = 1 its 3 waves a SIMD take a second group from 24,576
+// tets on, k_fused11's 2 of 16 elements from 32,768 on (us per stage k_fused11 /
+// k_quad, 24,576 tets 17.4 / 15.0, 27,030 18.5 / 19.7, 31,212 18.7 / 20.2, 32,832
+// 19.8 / 19.7, 36,936 24.8 / 20.7). At N = 4 up to 1,024 tets, one wave a SIMD of
+// k_fused11's, a stage is one group's chain of operations (162 tets 19.7 / 21.2,
+// 960 21.5 / 22.0, 1,080 24.3 / 21.6). Compressed registers leave k_quad in the
+// ranges of default_variant.
+int default_kcl_variant(int order, const StageArgs &a) {
+  const bool other = (order == 1 && a.n_elem > 24576 && a.n_elem <= 32768) || (order == 4 && a.n_elem <= 1024);
+  return a.variant == kQuadVariant && other ? 7 : a.variant;
+}
+
 void build_fused(rfhip_op *op, const rfhip_op_desc &d) {
   const int64_t K = d.n_elem;
   const int np = d.np, nfp = d.nfp, nf4 = 4 * nfp;
@@ -448,6 +462,7 @@ void build_fused(rfhip_op *op, const rfhip_op_desc &d) {
   a.quad_seq = has_quad_seq ? op->quad_seq.as<double>() : nullptr;
   a.quad_nodes = has_quad ? op->quad_nodes.p : nullptr;
   a.variant = default_variant(op->order, op->form, a);
+  op->kcl_variant = default_kcl_variant(op->order, a);
 }
 
 // ---- vectors at the boundary ---------------------------------------------
@@ -698,7 +713,9 @@ void kcl_impl(rfhip_op *op, void *ys, double dt, int64_t steps, int kind, int64_
     launch_copy(std64[0], ys, 8 * n, s);
   }
   const int nblk = weighted_err_blocks(n);
-  const int64_t nslot = fuse || fuse64 ? kcl_stage_slots(op->order, op->sa, fuse64) : 0;
+  StageArgs kcl = op->sa;
+  kcl.variant = op->kcl_variant;
+  const int64_t nslot = fuse || fuse64 ? kcl_stage_slots(op->order, kcl, fuse64) : 0;
   const int64_t npart = std::max<int64_t>(nblk, nslot);
   op->red.alloc(8 * (npart + 1));
   double *part = op->red.as<double>();
@@ -737,7 +754,7 @@ void kcl_impl(rfhip_op *op, void *ys, double dt, int64_t steps, int kind, int64_
       // pass also saves the starting y (kbak); the last one reduces the
       // error norm (session.rs:160-171) against it.
       for (int sg = 0; (fuse || fuse64) && sg < 5; ++sg) {
-        StageArgs a = op->sa;
+        StageArgs a = kcl;
         if (fuse64) {
           a.yin = std64[sc];
           a.yout = std64[1 - sc];
@@ -2067,7 +2084,7 @@ int rfhip_op_set_variant(rfhip_op *op, int variant) {
     if (!variant_available(op->order, op->form, variant, op->sa))
       throw Error{RFHIP_EUNSUPPORTED, "stage-kernel variant " + std::to_string(variant) +
                                           " cannot run on this operator (order or neighbour table)"};
-    op->sa.variant = variant;
+    op->sa.variant = op->kcl_variant = variant;
   });
 }
 
@@ -2139,6 +2156,7 @@ int rfhip_op_autotune(rfhip_op *op, int *chosen, double *ms_best) {
     for (int v = 0; v < nv; ++v)
       if (v_ms[v] < v_ms[best]) best = v;
     op->sa.variant = best;
+    op->kcl_variant = default_kcl_variant(op->order, op->sa);
     if (chosen) *chosen = best;
     if (ms_best) *ms_best = v_ms[best];
   });

@@ -250,6 +250,7 @@ struct rfhip_op {
   int kb_cap = 0;
   rfhip::DevOp dev{};
   rfhip::StageArgs sa{};  // fused forms: geometry part filled at creation
+  int kcl_variant = 0;  // stage-kernel variant of the fused KCL stages (set with sa.variant)
 };
 
 // CsrMatrix (rhs.rs:1575-1591) held in HBM: row_ptr n+1, col_idx and values
