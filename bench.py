@@ -94,7 +94,7 @@ def parse():
                     help="time the sparse state-space export (assemble_sparse) on the device instead of the "
                          "stepper: --sparse-cells box at --order, one JSON line in nonzeros/s")
     ap.add_argument("--krylov", action="store_true",
-                    help="time the Krylov exponential (expmv, FP64 Arnoldi with CGS2) on the --krylov-cells box "
+                    help="time the Krylov exponential (expmv, FP64 Arnoldi with DCGS2) on the --krylov-cells box "
                          "instead of the stepper: one JSON line in Arnoldi DOF-steps/s")
     ap.add_argument("--krylov-cells", type=int, nargs=3, default=[40, 30, 28])
     ap.add_argument("--krylov-dim", type=int, default=40)
@@ -130,13 +130,24 @@ def apply_bytes_per_dof(order: int) -> float:
     return 16.0 + 92.0 / (6 * np_)
 
 
+def krylov_bytes(order: int, n: int, dim: int) -> float:
+    """Algorithmic HBM bytes of one expmv call of `dim` columns without a stop
+    test, in vectors of n FP64 values: per column j the apply, one sweep of
+    inner products (k_gram2: the columns 0..j and the new product) and one
+    update (k_dcgs_update: the same j + 2 read, two written); then the
+    products that close the last column (dim + 1 read) and the combination
+    (dim read, one written)."""
+    vectors = sum((j + 2) + (j + 2) + 2 for j in range(dim)) + (dim + 1) + (dim + 1)
+    return 8.0 * n * vectors + dim * apply_bytes_per_dof(order) * n
+
+
 def krylov_bench(args) -> int:
     """expmv (fixed Arnoldi dimension m, no a-posteriori stop) on the stiff
     Krylov workload: the 201,600-tet N=3 unit box graded 20:1 toward a thin
     slab (eps_r 10, sigma 50), pulse field, t = 3 / rho (rho from 20 power
     iterations of the apply, so ||tA|| is about 3). Unit: one Arnoldi
-    DOF-step = one basis vector entry of one Arnoldi step (apply + two CGS2
-    passes)."""
+    DOF-step = one basis vector entry of one Arnoldi step (apply, products
+    and update)."""
     import numpy as np
 
     import rapidfem_amd as R
@@ -168,21 +179,9 @@ def krylov_bench(args) -> int:
     ms = float(np.median(times))
     wall = float(np.median(walls))
     dim = g.last_dim
-    # algorithmic HBM bytes of the whole call: per step j (cols = j + 1 basis
-    # vectors) the apply, three sweeps of the two-pass Gram-Schmidt (the
-    # projections read cols + 1 vectors; the first update fused with the
-    # second projections reads cols + 1 and writes 1; the second update
-    # reads cols + 1 and writes 1) and the normalisation (read w, write the
-    # next basis vector); plus the start (norm, scale) and the final
-    # combination (reads dim vectors, writes one)
-    b = 3 * 8.0 * n + (dim + 1) * 8.0 * n
-    for j in range(dim):
-        cols = j + 1
-        b += apply_bytes_per_dof(args.order) * n + (3 * cols + 5) * 8.0 * n
-        if j + 1 < dim:
-            b += 16.0 * n
+    b = krylov_bytes(args.order, n, dim)
     gbs = b / (ms * 1e-3) / 1e9
-    out = {"metric": "Krylov exponential (expmv, CGS2 Arnoldi) DOF-steps/s", "value": n * dim / (ms * 1e-3),
+    out = {"metric": "Krylov exponential (expmv, DCGS2 Arnoldi) DOF-steps/s", "value": n * dim / (ms * 1e-3),
            "unit": "Arnoldi DOF-steps/s", "n_gpus": 1, "reps": len(times), "higher_is_better": True,
            "dtype": "f64", "data": "synthetic", "ms_per_call": ms, "ms_per_arnoldi_step": ms / dim,
            "host_inclusive": {"ms_per_call": wall, "value": n * dim / (wall * 1e-3),
@@ -194,8 +193,8 @@ def krylov_bench(args) -> int:
            "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None,
                         "algorithmic_bytes_per_call": b,
-                        "kernel": "whole call (apply + k_multi_dot + k_axpy_dot + k_axpy_basis_norm + scale + lincomb), "
-                                  "host round trip per CGS2 pass included"}}
+                        "kernel": "whole call (apply + k_gram2 + k_dcgs_update per column, k_multi_dot, k_lincomb), "
+                                  "one host round trip per column included"}}
     if not args.no_cpu:
         from oracle import oracle as O
 
@@ -319,7 +318,7 @@ def proposer_bench(args) -> int:
     gain = res["plain"]["device_ms"] / res["learned"]["device_ms"]
     out = {"metric": "Krylov-exp wall time, learned (h, m) proposer vs plain controller at equal tolerance",
            "value": round(gain, 3), "unit": "x (plain ms / learned ms)", "n_gpus": 1, "higher_is_better": True,
-           "dtype": "f64 (Arnoldi, CGS2, Pade-13), f32 network", "data": "synthetic", "tol": tol,
+           "dtype": "f64 (Arnoldi, DCGS2, Pade-13), f32 network", "data": "synthetic", "tol": tol,
            "plain": res["plain"], "learned": res["learned"], "fine": {"steps": int(len(sf)), "tol": tol * 1e-3},
            "compressed_basis": comp, "cost_model_ms": cost, "plain_fixed_m": sweep,
            # the plain controller at the dimension that was best in hindsight on this workload
@@ -446,7 +445,7 @@ def kcl_bench(args) -> int:
     gc.set_kcl_registers("compressed")
     runs_c, y_c = reps(gc, "compressed registers, fused update")
     compressed = summary("compressed registers, fused update", runs_c, y_c)
-    compressed["update"] = "in the stage kernel's epilogue (k_fused11, no k stored)"
+    compressed["update"] = "in the stage kernel's epilogue (k_quad or k_fused11, no k stored)"
     compressed["separate_update"] = separate
     compressed["rel_l2_vs_separate_update"] = float(np.linalg.norm(y_c - y_s) / np.linalg.norm(y_s))
     compressed["speedup_vs_separate_update"] = separate["ms_per_substep"] / compressed["ms_per_substep"]
@@ -461,7 +460,7 @@ def kcl_bench(args) -> int:
            "unit": "DOF-stage/s", "n_gpus": 1, "reps": len(runs), "higher_is_better": True, "dtype": "f64",
            "data": "synthetic", "ms_per_call": ms, "substeps": sub, "accepted": acc, "rejected": rej,
            "ms_per_substep": ms / max(sub, 1),
-           "update": "in the stage kernel's epilogue where the operator allows it (k_fused11)",
+           "update": "in the stage kernel's epilogue where the operator allows it (k_quad or k_fused11)",
            "separate_update": f64_separate, "compressed_registers": compressed,
            "host_inclusive": {"ms_per_call": wall, "value": n * 5 * sub / (wall * 1e-3),
                               "note": "the whole call: state upload, layout conversions and the 3 frames "
