@@ -165,28 +165,32 @@ void build_plain(rfhip_op *op, const rfhip_op_desc &d) {
   dv.port = op->port.as<int>();
   dv.perm = op->perm.as<int>();
 }
-// Stage-kernel variant an operator starts with: k_quad (variant 9) where its
-// tables exist, the fastest on MI355X at every order and both register layouts
-// but for the ranges named below. us per stage, fastest other variant
-// against k_quad, N = 1..4: FP64 registers, 1,296 tets 5.6 / 3.9, 7.6 / 5.4,
-// 9.4 / 8.4, 15.4 / 15.1; 1.3M / 768k / 324k / 384k tets 288 / 271, 484 / 350,
-// 416 / 290, 1232 / 690; compressed registers, the same large meshes 235 / 221,
-// 410 / 306, 376 / 262, 1170 / 735, with the same bits as the variants named
-// below (their rounding of p to f32 turns any other order of the sums into
-// differences of its own size within a few dozen stages). Compressed registers
-// on small meshes at N = 3, 4, where a stage is one group's chain of operations
-// and that order makes it longer, stay with those variants (1,296 tets: 9.6 /
-// 10.0 and 16.7 / 19.6 us; 2,688: 10.1 / 10.3 and 19.4 / 19.3; 3,072: 10.3 / 10.3
-// and 20.8 / 19.4; 6,000: 14.0 / 11.6 and 33.0 / 22.1), and so do they at N = 1
-// in a range that the sweep shows and nothing yet explains: 24,576 tets 8.0 /
-// 7.8, 26,112 8.1 / 8.8, 31,212 8.4 / 8.9, 45,600 13.2 / 14.0, 66,792 15.1 /
-// 15.5, then 101,400 22.5 / 21.6. Operators without
-// the tables (no permuted node tables, or a state of 2^32 bytes and more) start
-// with the fastest of the rest. autotune re-picks on the operator's own mesh.
+// Stage-kernel variant an operator starts with, from LSERK4 stages on MI355X:
+// k_quad (variant 9) where its tables exist, the fastest at every order with
+// FP64 registers, and with compressed ones but for the ranges named below. us
+// per stage, fastest other variant against k_quad, N = 1..4: FP64 registers,
+// 1,296 tets 6.7 / 4.6, 7.7 / 5.7, 9.4 / 8.4, 16.9 / 15.3; 1.3M / 768k / 324k /
+// 384k tets 288 / 269, 484 / 350, 416 / 290, 1232 / 690; compressed registers,
+// the same large meshes 235 / 221, 410 / 306, 376 / 262, 1170 / 735, with the
+// same bits as the variants named below (their rounding of p to f32 turns any
+// other order of the sums into differences of its own size within a few dozen
+// stages). Compressed registers stay with those variants on small meshes at N =
+// 3, 4, where a stage is one group's chain of operations and that order makes it
+// longer (1,296 tets: 9.6 / 10.0 and 16.7 / 19.6 us; 2,688: 10.1 / 10.3 and 19.4 /
+// 19.4; 3,072: 10.3 / 10.3 and 20.7 / 19.5; 6,000: 14.0 / 11.6 and 33.0 / 22.0),
+// and at N = 1 in a range where either wins by up to a tenth as the last wave of
+// one or the other is full or nearly empty (24,576 tets 8.0 / 7.6, 26,112 8.1 /
+// 8.6, 29,478 10.3 / 9.2, 45,600 13.3 / 13.5, 66,792 15.3 / 15.3, then 101,400 23.2 /
+// 22.1). Operators without the tables (no permuted node tables, or a state of
+// 2^32 bytes and more) start with the fastest of the rest. The applies of a
+// compressed operator run its variant too. autotune re-picks on the operator's
+// own mesh.
 int default_variant(int order, int form, const StageArgs &a) {
   if (form_vmf(form)) return 1;
   const bool c = form == RFHIP_FORM_FUSED_F64C;
-  const bool keep = c && (order == 1 ? a.n_elem > 24576 && a.n_elem < 70000 : order == 3 ? a.n_elem < 3200 : order == 4 && a.n_elem < 2560);
+  const bool keep = c && (order == 1   ? a.n_elem > 24576 && a.n_elem < 70000
+                          : order == 3 ? a.n_elem < 3200
+                                       : order == 4 && a.n_elem < 2560);
   if (!keep && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
   switch (order) {
     case 1: return c ? 7 : 5;

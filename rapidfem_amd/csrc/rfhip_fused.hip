@@ -89,8 +89,9 @@ __device__ __forceinline__ void load_trace(const StageArgs &io, int64_t nb, doub
 
 // EPI: 0 = apply (dy = A y, FP64), 1 = LSERK stage with FP64 registers,
 // 2 = LSERK stage with compressed registers (y f32+bf16, p f32), 3 = KCL
-// stage with compressed registers (k_fused11 only, node_kcl), 4 = KCL stage
-// with FP64 registers (k_fused11 only, node_kcl64).
+// stage with compressed registers (here k_fused11 only, node_kcl), 4 = KCL
+// stage with FP64 registers (here k_fused11 only, node_kcl64); k_quad
+// (rfhip_quad.hip) has them all.
 //
 // KCL stage update of one node with compressed registers
 // (explicit_adaptive.rs:107-149), the same arithmetic as the separate pass

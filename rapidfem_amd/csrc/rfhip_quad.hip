@@ -20,7 +20,7 @@
 //  * D_k is sparse on equispaced nodes: 4x4 blocks of D_k that are zero are
 //    left out at compile time, and the node groups below are the ones an
 //    annealed search found to leave the fewest: 20 of 27, 49 of 75 and 138 of
-//    243 blocks at N = 2, 3, 4 (24 % to 43 % of the volume products).
+//    243 blocks at N = 2, 3, 4 (26 % to 43 % of the volume products).
 //  * state in and stage update out are linear over the group (16-byte or
 //    8 + 4 byte loads and stores per lane, no lane idle): y goes to LDS as FP64,
 //    and the right-hand side comes back through the same LDS.
@@ -38,9 +38,9 @@
 // against 416 for the variant before it): the memory side. Leaving out all
 // products changes nothing, streaming the state and p alone takes 245 us (5.3
 // TB/s), the neighbour traces, 10 M line requests to L2, the rest. At N = 4
-// (384,000 tets, 690 us against 1232) products and vector instructions fill
-// about 70 % of the issue cycles. Compressed registers: 262 us against 376 and
-// 735 against 1170, bound the same way.
+// (384,000 tets, 690 us against 1232) products and vector instructions fill 47
+// and 20 % of the issue cycles. Compressed registers: 262 us against 376 and 735
+// against 1170, bound the same way (49 and 28 %).
 #include <algorithm>
 #include <map>
 #include <mutex>
