@@ -188,9 +188,7 @@ void build_plain(rfhip_op *op, const rfhip_op_desc &d) {
 int default_variant(int order, int form, const StageArgs &a) {
   if (form_vmf(form)) return 1;
   const bool c = form == RFHIP_FORM_FUSED_F64C;
-  const bool keep = c && (order == 1   ? a.n_elem > 24576 && a.n_elem < 70000
-                          : order == 3 ? a.n_elem < 3200
-                                       : order == 4 && a.n_elem < 2560);
+  const bool keep = c && (order >= 3 ? a.n_elem < 2560 : order == 1 && a.n_elem > 24576 && a.n_elem < 70000);
   if (!keep && variant_available(order, form, kQuadVariant, a)) return kQuadVariant;
   switch (order) {
     case 1: return c ? 7 : 5;
